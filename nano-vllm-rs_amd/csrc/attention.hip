@@ -827,7 +827,10 @@ extern "C" int nv_attention(nv_context* c, const void* q, const void* kc, const 
     // The ordered kernels index cache rows in int32.
     const bool vec = nvr::aligned(q, 16) && nvr::aligned(kc, 16) && nvr::aligned(vc, 16) &&
                      int64_t(blocks) * bs <= 0x7fffffff;
-    if (vec && dim == 128)
+    if (vec && nvr::aligned(out, 16) && nvr::attention_tiles_fit(rows, qh, kvh, dim, bs, batch))
+        nvr::launch_attention_tiles(c, q16, k16, v16, p32, s32, t32, o16, rows, qh, kvh, bs, blocks, stride, batch,
+                                    max_context);
+    else if (vec && dim == 128)
         launch_dim<128>(c, q16, k16, v16, p32, s32, t32, o16, rows, qh, kvh, bs, blocks, stride, batch, max_context);
     else if (vec && dim == 64)
         launch_dim<64>(c, q16, k16, v16, p32, s32, t32, o16, rows, qh, kvh, bs, blocks, stride, batch, max_context);

@@ -1,0 +1,333 @@
+// Paged causal GQA attention over tiles of 16 (token, q head) rows on the fp32
+// matrix instructions: the prefill form of nv_attention (attention.hip states
+// the semantics and the fp32 order; this file keeps both bit for bit).
+//
+// v_mfma_f32_16x16x4_f32 computes D = C + A B as four chained fused
+// multiply-adds in k order, subnormals kept (checked on MI355X over 2.5 M
+// outputs, normal, widely scaled and subnormal, against host fmaf chains: no
+// mismatch; the reverse order mismatches in half of them). So the two chains
+// that the reference's order prescribes are matrix products:
+//   - dot chain c (d = c, c + 32, c + 64, c + 96) of 16 tokens x 16 rows is one
+//     instruction with k = the four d's and C = 0; the 32-lane tree over the
+//     chains is 31 adds of the results;
+//   - the value chain over tokens is a sequence of instructions whose k runs
+//     over four consecutive tokens, accumulating in place.
+// The matrix form has the FMA rate of the plain VALU on this GPU (both 34
+// cycles per 1024 FMAs, and they do not overlap); what it removes is the rest:
+// a row-by-row kernel reads every K and V row from LDS and widens it once per
+// query row, here once per 16.
+//
+// Layout. A block of four waves owns 16 rows: TR = 16 >> hg_shift consecutive
+// batch rows x HG = 1 << hg_shift q heads of one kv head. Rows of several
+// sequences are processed one sequence at a time (the others masked).
+//   1. Scores, transposed (M = tokens, N = rows): wave w takes tiles of 16
+//      tokens 2w, 2w + 1, 2w + 8, 2w + 9, ... Lane (m, j) holds 64 contiguous
+//      bytes of token tok(m) = 4 (m % 4) + m / 4, d = 32 j .. 32 j + 31: the A
+//      operands of all 32 chains. The permuted tokens make result register r
+//      of lane group a the score of token 4 r + a, which is the operand layout
+//      of phase 3 as it stands. The first kChunk tiles' scores go to LDS.
+//   2. Row maxima; p = exp(score - max). A wave's tiles 2w, 2w + 1 (mod 16) are
+//      threads 32 w .. 32 w + 31 and 128 + 32 w .. of the reference's block
+//      sum, so the sum's chains and its first five levels stay in the wave.
+//   3. Values, transposed (M = d, N = rows): wave w takes d = 32 w .. 32 w + 31
+//      of every tile, d = 32 w + 2 m + e in instruction e.
+// Contexts longer than a chunk (64 tiles) score the later chunks a second time
+// in phase 2 rather than keep them.
+//
+// Measured on MI355X against one block per row (attention.hip): 8 prompts of
+// 1024 rows in all 80.4 -> 33.3 us, one 1021-token prompt 280 -> 82 us, 1024
+// rows at positions 3072 .. 4095 1627 -> 560 us (54 TFLOP/s of the 140 that the
+// fp32 FMAs reach; the rest is the tree, the exponentials and the second
+// scoring of long contexts).
+//
+// Masked tokens may hold anything (an Inf or NaN times a zero p, or a -0 sum,
+// must not change a row that does not see them), so tiles that some row sees
+// only in part run their value chains on the VALU with the row's own mask.
+#include "../../include/nano_hip.h"
+#include "nvr_device.h"
+#include "nvr_internal.h"
+
+namespace {
+
+using nvr::kWave;
+typedef float f32x4_t __attribute__((ext_vector_type(4)));
+
+constexpr int kThreads = 256, kWaves = 4;
+constexpr int kDim = 128;
+constexpr int kRows = 16;    // (token, head) rows per block
+constexpr int kTokens = 16;  // tokens per tile
+constexpr int kChunk = 64;   // tiles whose probabilities LDS holds (64 KB: two blocks per CU)
+constexpr int kMaxTiles = 4096 / kTokens;
+
+__device__ __forceinline__ f32x4_t mfma(float a, float b, f32x4_t c) {
+    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+}
+
+__global__ __launch_bounds__(kThreads, 2) void attention_tiles(
+    const uint16_t* __restrict__ q, const uint16_t* __restrict__ kc, const uint16_t* __restrict__ vc,
+    const int* __restrict__ positions, const int* __restrict__ seqs, const int* __restrict__ tables,
+    uint16_t* __restrict__ out, int rows, int qh, int kvh, int bs, int blocks, int stride, int batch, int max_context,
+    int hg_shift, int row_tiles) {
+    extern __shared__ __align__(16) unsigned char smem[];
+    f32x4_t* probs = reinterpret_cast<f32x4_t*>(smem);  // [kChunk][64 lanes]
+    __shared__ int tile_row[kMaxTiles];                 // physical token row of each tile's first token, or -1
+    __shared__ float red_max[kWaves][kRows];
+    __shared__ float red_sum[2 * kWaves][kRows];
+
+    const int lane = threadIdx.x & (kWave - 1), wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+    const int n = lane & 15, a = lane >> 4;  // row of the tile; lane group
+    // Consecutive blocks take the head groups of one row tile, so each XCD
+    // (blocks go round the eight) sees few kv heads and keeps their K and V in
+    // its L2; the last rows, whose contexts are the longest, start first.
+    const int groups = qh >> hg_shift;
+    const int group = int(blockIdx.x) % groups, tile = row_tiles - 1 - int(blockIdx.x) / groups;
+    const int head = (group << hg_shift) + (n & ((1 << hg_shift) - 1));
+    const int kvhead = (group << hg_shift) / (qh / kvh);
+    const int row = tile * (kRows >> hg_shift) + (n >> hg_shift);
+    const bool exists = row < rows;
+    const int seq_n = exists ? seqs[row] : -1;
+    const int64_t ctx64 = exists ? int64_t(positions[row]) + 1 : 0;
+    const bool valid = exists && seq_n >= 0 && seq_n < batch && ctx64 >= 1 && ctx64 <= max_context &&
+                       ctx64 <= int64_t(stride) * bs;
+    const int64_t row_head = int64_t(exists ? row : 0) * qh + head;
+    uint16_t* dst = out + row_head * kDim + 32 * wave + 8 * a;
+    if (exists && !valid) *reinterpret_cast<uint4*>(dst) = make_uint4(0, 0, 0, 0);
+
+    float qf[32];  // q[32 a + c]: operand B of chain c
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+        nvr::unpack8(*reinterpret_cast<const uint4*>(q + row_head * kDim + 32 * a + 8 * i), qf + 8 * i);
+    const float kScale = 1.0f / sqrtf(float(kDim));
+    const int64_t token_stride = int64_t(kvh) * kDim;
+    const uint16_t* kcol = kc + int64_t(kvhead) * kDim;
+    const uint16_t* vcol = vc + int64_t(kvhead) * kDim;
+    const int klane = (4 * (n & 3) + (n >> 2)) * int(token_stride) + 32 * a;
+
+    uint32_t todo = uint32_t(__ballot(valid)) & 0xffffu;  // rows still to do (the same in every wave)
+    while (todo != 0) {
+        const int seq = __builtin_amdgcn_readlane(seq_n, __builtin_ctz(todo));
+        const bool active = valid && seq_n == seq;
+        todo &= ~uint32_t(__ballot(active));
+        const int ctx = active ? int(ctx64) : 0;
+        int hi = ctx, lo = active ? ctx : max_context;
+#pragma unroll
+        for (int o = 1; o < kRows; o <<= 1) {
+            hi = max(hi, nvr::xor_lane(hi, o));
+            lo = min(lo, nvr::xor_lane(lo, o));
+        }
+        const int ctx_max = __builtin_amdgcn_readfirstlane(hi), ctx_min = __builtin_amdgcn_readfirstlane(lo);
+        const int tiles = (ctx_max + kTokens - 1) / kTokens, full = ctx_min / kTokens;
+        if (int(threadIdx.x) < tiles) {
+            const int t0 = int(threadIdx.x) * kTokens, lb = t0 / bs;
+            const int e = tables[int64_t(seq) * stride + lb];
+            tile_row[threadIdx.x] = e >= 0 && e < blocks ? e * bs + (t0 - lb * bs) : -1;
+        }
+        __syncthreads();
+
+        // Tiles past the context or in an invalid block load the first rows
+        // of block 0; their scores are masked and their values skipped.
+        auto place = [&](int t) { return __builtin_amdgcn_readfirstlane(tile_row[min(t, tiles - 1)]); };
+        auto load_k = [&](uint4 (&kb)[4], int t) {
+            const uint16_t* base = kcol + int64_t(max(place(t), 0)) * token_stride;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) kb[i] = *reinterpret_cast<const uint4*>(base + klane + 8 * i);
+        };
+        auto scores = [&](const uint4 (&kb)[4], int t) -> f32x4_t {
+            const uint32_t* w = reinterpret_cast<const uint32_t*>(kb);
+            auto chain = [&](int c) {
+                return mfma(c & 1 ? nvr::bf16_hi(w[c >> 1]) : nvr::bf16_lo(w[c >> 1]), qf[c], f32x4_t{0, 0, 0, 0});
+            };
+            auto l16 = [&](int c) { return chain(c) + chain(c + 16); };
+            auto l8 = [&](int c) { return l16(c) + l16(c + 8); };
+            auto l4 = [&](int c) { return l8(c) + l8(c + 4); };
+            auto l2 = [&](int c) { return l4(c) + l4(c + 2); };
+            const f32x4_t dot = l2(0) + l2(1);
+            const bool ok = place(t) >= 0;
+            f32x4_t s;
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+                s[r] = ok && t * kTokens + 4 * r + a < ctx ? dot[r] * kScale : -__builtin_inff();
+            return s;
+        };
+        // Wave-tile s of this wave: pairs 2w, 2w + 1 of every eight tiles.
+        auto tile_of = [&](int s) { return 8 * (s >> 1) + 2 * wave + (s & 1); };
+
+        // ---- 1. scores and row maxima ----
+        float m = -__builtin_inff();
+        {
+            uint4 kA[4], kB[4];
+            load_k(kA, tile_of(0));
+            load_k(kB, tile_of(1));
+            auto step = [&](uint4 (&kb)[4], int s) {
+                const int t = tile_of(s);
+                const f32x4_t sc = scores(kb, t);
+                load_k(kb, tile_of(s + 2));
+#pragma unroll
+                for (int r = 0; r < 4; ++r) m = fmaxf(m, sc[r]);
+                if (t < kChunk) probs[t * kWave + lane] = sc;
+            };
+            for (int s = 0; tile_of(s) < tiles; s += 2) {
+                step(kA, s);
+                if (tile_of(s + 1) < tiles) step(kB, s + 1);
+            }
+        }
+        m = fmaxf(m, nvr::xor_lane(m, 16));
+        m = fmaxf(m, nvr::xor_lane(m, 32));
+        if (a == 0) red_max[wave][n] = m;
+        __syncthreads();
+        m = fmaxf(fmaxf(red_max[0][n], red_max[1][n]), fmaxf(red_max[2][n], red_max[3][n]));
+        const bool finite = __builtin_isfinite(m);
+
+        float sums[2][2][4] = {};           // the reference's thread sums of this wave's tiles (mod 16)
+        f32x4_t o0 = {0, 0, 0, 0}, o1 = {0, 0, 0, 0};
+        for (int c0 = 0; c0 < tiles; c0 += kChunk) {
+            const int c1 = min(tiles, c0 + kChunk);
+            // ---- 2. probabilities of the chunk ----
+            auto prob = [&](f32x4_t sc, int t, float (&sum)[4]) {
+                f32x4_t p;
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    p[r] = finite ? nvr::nvr_expf(sc[r] - m) : 0.0f;
+                    sum[r] += p[r];
+                }
+                probs[(t - c0) * kWave + lane] = p;
+            };
+            if (c0 == 0) {
+                for (int s = 0; tile_of(s) < c1; s += 4) {
+#pragma unroll
+                    for (int u = 0; u < 4; ++u) {
+                        const int t = tile_of(s + u);
+                        if (t < c1) prob(probs[t * kWave + lane], t, sums[u >> 1][u & 1]);
+                    }
+                }
+            } else {
+                const int s0 = c0 / kWaves;
+                uint4 kA[4], kB[4];
+                load_k(kA, tile_of(s0));
+                load_k(kB, tile_of(s0 + 1));
+                for (int s = s0; tile_of(s) < c1; s += 4) {
+#pragma unroll
+                    for (int u = 0; u < 4; ++u) {
+                        const int t = tile_of(s + u);
+                        uint4(&kb)[4] = u & 1 ? kB : kA;
+                        if (t < c1) {
+                            const f32x4_t sc = scores(kb, t);
+                            load_k(kb, tile_of(s + u + 2));
+                            prob(sc, t, sums[u >> 1][u & 1]);
+                        }
+                    }
+                }
+            }
+            __syncthreads();
+
+            // ---- 3. values of the chunk ----
+            const int f1 = min(full, c1);
+            auto load_v = [&](uint32_t (&v)[4], int t) {
+                const uint16_t* base = vcol + int64_t(max(place(t), 0)) * token_stride + 32 * wave + 2 * n;
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+                    v[r] = *reinterpret_cast<const uint32_t*>(base + (4 * r + a) * int(token_stride));
+            };
+            auto values = [&](const uint32_t (&v)[4], int t) {
+                if (place(t) < 0) return;  // an invalid block adds no term
+                const f32x4_t p = probs[(t - c0) * kWave + lane];
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    o0 = mfma(nvr::bf16_lo(v[r]), p[r], o0);
+                    o1 = mfma(nvr::bf16_hi(v[r]), p[r], o1);
+                }
+            };
+            if (c0 < f1) {
+                uint32_t vA[4], vB[4], vC[4], vD[4];
+                load_v(vA, c0);
+                load_v(vB, c0 + 1);
+                load_v(vC, c0 + 2);
+                for (int t = c0; t < f1; t += 4) {
+                    load_v(vD, t + 3);
+                    values(vA, t);
+                    load_v(vA, t + 4);
+                    if (t + 1 < f1) values(vB, t + 1);
+                    load_v(vB, t + 5);
+                    if (t + 2 < f1) values(vC, t + 2);
+                    load_v(vC, t + 6);
+                    if (t + 3 < f1) values(vD, t + 3);
+                }
+            }
+            // Tiles that some row sees in part: token by token, each row masked by its own context.
+            for (int t = max(full, c0); t < c1; ++t) {
+                const int ph = place(t);
+                if (ph < 0) continue;
+                const uint16_t* base = vcol + int64_t(ph) * token_stride + 32 * wave + 8 * a;
+                uint4 v[kTokens];
+#pragma unroll
+                for (int i = 0; i < kTokens; ++i) v[i] = *reinterpret_cast<const uint4*>(base + i * int(token_stride));
+                const float* pt = reinterpret_cast<const float*>(probs + (t - c0) * kWave);
+#pragma unroll
+                for (int i = 0; i < kTokens; ++i) {
+                    if (t * kTokens + i >= ctx_max) break;  // uniform
+                    const float p = pt[(16 * (i & 3) + n) * 4 + (i >> 2)];
+                    const bool sees = t * kTokens + i < ctx;
+                    float f[8];
+                    nvr::unpack8(v[i], f);
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        const float x = __builtin_fmaf(p, f[2 * r], o0[r]), y = __builtin_fmaf(p, f[2 * r + 1], o1[r]);
+                        o0[r] = sees ? x : o0[r];
+                        o1[r] = sees ? y : o1[r];
+                    }
+                }
+            }
+            if (c1 < tiles) __syncthreads();  // the next chunk overwrites the probabilities
+        }
+
+        // ---- 4. the block sum's tree and the output ----
+        // Tile pair (2w, 2w + 1): offset 16 between the two tiles, 8 and 4
+        // between registers r, 2 and 1 between lane groups a.
+#pragma unroll
+        for (int g = 0; g < 2; ++g) {
+            float x[4];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) x[r] = sums[g][0][r] + sums[g][1][r];
+            float s = (x[0] + x[2]) + (x[1] + x[3]);
+            s += nvr::xor_lane(s, 32);
+            s += nvr::xor_lane(s, 16);
+            if (a == 0) red_sum[4 * g + wave][n] = s;
+        }
+        __syncthreads();
+        const float den = ((red_sum[0][n] + red_sum[4][n]) + (red_sum[2][n] + red_sum[6][n])) +
+                          ((red_sum[1][n] + red_sum[5][n]) + (red_sum[3][n] + red_sum[7][n]));
+        float o[8];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            o[2 * r] = den > 0.0f ? o0[r] / den : 0.0f;
+            o[2 * r + 1] = den > 0.0f ? o1[r] / den : 0.0f;
+        }
+        if (active) *reinterpret_cast<uint4*>(dst) = nvr::pack8(o);
+        if (todo != 0) __syncthreads();  // the next sequence reuses the LDS arrays
+    }
+}
+
+}  // namespace
+
+namespace nvr {
+
+// Rows of one sequence share a tile's K and V; a batch of one row per sequence
+// would leave 15 of 16 rows masked and walk its sequences one after the other,
+// so the batch must average at least four rows a sequence.
+bool attention_tiles_fit(int rows, int qh, int kvh, int dim, int bs, int batch) {
+    return dim == kDim && bs % kTokens == 0 && rows >= 4 * int64_t(batch) && int64_t(rows) * qh < (int64_t(1) << 31);
+}
+
+void launch_attention_tiles(nv_context* c, const uint16_t* q, const uint16_t* k, const uint16_t* v, const int* p,
+                            const int* s, const int* t, uint16_t* o, int rows, int qh, int kvh, int bs, int blocks,
+                            int stride, int batch, int max_context) {
+    const int ratio = qh / kvh;
+    int shift = 0;
+    while (shift < 4 && ratio % (2 << shift) == 0) ++shift;
+    const int per = kRows >> shift, row_tiles = (rows + per - 1) / per;
+    hipLaunchKernelGGL(attention_tiles, dim3(unsigned(row_tiles) * unsigned(qh >> shift)), dim3(kThreads),
+                       sizeof(f32x4_t) * kChunk * kWave, c->stream, q, k, v, p, s, t, o, rows, qh, kvh, bs, blocks,
+                       stride, batch, max_context, shift, row_tiles);
+}
+
+}  // namespace nvr

@@ -1,0 +1,77 @@
+"""nv_attention's tile form (several rows per sequence, head dim 128, blocks of
+whole 16-token tiles) against the oracle, bit for bit: head groups, block
+sizes, edges of tiles and of the 1024-token chunks, tiles that hold rows of
+several sequences, invalid rows and blocks, and values that a masked token
+must not let through."""
+import numpy as np
+import pytest
+
+import oracle as ora
+from helpers import assert_bits_equal
+from test_gpu_kernels import _attention, _attention_case
+
+pytestmark = pytest.mark.gpu
+
+
+def _rows(spans):
+    """Flattened (positions, sequence ids) of sequences that add tokens [first, first + n)."""
+    return (np.concatenate([np.arange(first, first + n) for first, n in spans]),
+            np.concatenate([np.full(n, i) for i, (_, n) in enumerate(spans)]))
+
+
+@pytest.mark.parametrize("qh,kvh", [(1, 1), (2, 2), (4, 2), (6, 2), (8, 2), (16, 2), (16, 1), (12, 2), (32, 1)])
+@pytest.mark.parametrize("bs", [16, 48, 256])
+def test_tiles_head_groups_and_block_sizes(gpu, qh, kvh, bs):
+    """1, 2, 4, 8 and 16 q heads of a kv head per tile (also ratios 3, 6 and 32);
+    prompts of 1, 37 and 150 tokens, so tiles hold rows of two or three sequences."""
+    pos, seqs = _rows([(0, 37), (0, 1), (0, 150), (29, 5)])
+    _attention_case(gpu, 300 + qh + bs, pos, seqs, qh, kvh, 128, bs, 4, -(-160 // bs), 160)
+
+
+@pytest.mark.parametrize("first,n", [(0, 16), (0, 17), (15, 9), (1007, 40), (1023, 1), (1016, 8), (2040, 24), (4079, 17)])
+def test_tiles_context_edges(gpu, first, n):
+    """Contexts that end on, before and after the edges of 16-token tiles and of
+    the 64-tile chunks, up to the longest context."""
+    pos, seqs = _rows([(first, n)])
+    pos, seqs = np.tile(pos, max(1, -(-4 // n))), np.tile(seqs, max(1, -(-4 // n)))
+    _attention_case(gpu, 330 + n, pos, seqs, 4, 2, 128, 256, 1, 16, 4096)
+
+
+def test_tiles_rows_in_any_order(gpu):
+    """Rows of three sequences interleaved and out of order, decode rows among them."""
+    rng = np.random.default_rng(350)
+    pos, seqs = rng.integers(0, 500, size=67), rng.integers(0, 3, size=67)
+    _attention_case(gpu, 351, pos, seqs, 4, 2, 128, 64, 3, 8, 512, q_std=6.0)
+
+
+def test_tiles_invalid_rows_and_blocks(gpu):
+    """Bad sequence ids and contexts give zero rows; table entries outside the
+    cache drop their tokens, also in a row's last block."""
+    stride, bs = 4, 64
+    pos, seqs = _rows([(180, 40), (30, 40), (0, 64)])
+    seqs[5], seqs[41], pos[7], pos[50] = -1, 3, 256, -1
+    holes = [(1, -1), (3, 3 * stride), (stride + 1, -9), (2 * stride, 3 * stride + 4)]
+    want = _attention_case(gpu, 360, pos, seqs, 4, 2, 128, bs, 3, stride, 256, holes=holes)
+    assert not want[[5, 7, 41, 50]].any()
+
+
+def test_tiles_masked_tokens_do_not_leak(gpu):
+    """V rows of Inf, NaN and values whose products round to -0 right after a
+    row's context, NaN and Inf keys, and underflowing probabilities: each row
+    equals the oracle, which never reads past the context."""
+    qh, kvh, dim, bs, blocks, rows = 4, 2, 128, 16, 8, 48
+    q = ora.normal_bf16((rows, qh, dim), 371, 0.0, 6.0)
+    kc = ora.normal_bf16((blocks, bs, kvh, dim), 372, 0.0, 1.0)
+    vc = ora.normal_bf16((blocks, bs, kvh, dim), 373, 0.0, 1.0)
+    flat = vc.reshape(blocks * bs, kvh, dim)  # the first row's context is tokens 0 .. 36: its sum there is -0
+    flat[:37, :, 16:24], flat[0, :, 16:24], flat[37:, :, 16:24] = 0x8000, 0x8001, 0x3F80
+    vc[3, 0, :, 40:48], vc[3, 5, :, 48:52], vc[3, 9, :, 52:56] = 0x7F80, 0xFF80, 0x7FC0
+    kc[4, 3, 0, 7], kc[4, 5, 1, 9] = 0x7FC0, 0x7F80
+    tables = np.arange(blocks, dtype=np.int32)
+    pos, seqs = (np.arange(rows) + 36).astype(np.int32), np.zeros(rows, np.int32)
+    want = ora.attention(q, kc, vc, pos, seqs, tables, rows, qh, kvh, dim, bs, blocks, blocks, 1, 128)
+    got = _attention(gpu, q, kc, vc, pos, seqs, tables, rows, qh, kvh, dim, bs, blocks, blocks, 1, 128)
+    nan = (want & 0x7FFF) > 0x7F80
+    assert nan.any() and (want == 0x8000).any() and ((want & 0x7FFF) == 0x7F80).any()
+    assert np.array_equal(nan, (got & 0x7FFF) > 0x7F80)  # a NaN's sign and payload are not specified
+    assert_bits_equal(np.where(nan, 0, got), np.where(nan, 0, want))
