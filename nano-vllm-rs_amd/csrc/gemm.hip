@@ -261,10 +261,10 @@ void launch_rows(nv_context* c, const uint16_t* x, const uint16_t* res, uint16_t
 // A block of WAVES waves owns a column tile of 16 and splits k over its
 // waves; each wave loads its W and X pieces straight into the MFMA operand
 // layouts (rows >= m read row m - 1 and are zeroed), all before the first
-// MFMA, and the partial tiles are summed through LDS in wave order. 4-wave
-// blocks serve wide outputs; outputs with fewer 16-column tiles than CUs take
-// gemm_narrow below 17 rows and 16-wave blocks (each streaming its tile's
-// whole k with 16 waves of loads in flight) from 17 rows.
+// MFMA, and the partial tiles are summed through LDS in wave order. It serves
+// what neither gemm_narrow (fewer 16-column tiles than CUs, at most 16 rows)
+// nor gemm_stream (at least as many tiles, k 1024 or 2048) takes, with 16 waves
+// of loads in flight per tile.
 template <int WAVES, int STEPS, int MT>
 __global__ __launch_bounds__(WAVES * 64) void gemm_rows(const uint16_t* __restrict__ x,
                                                         const uint16_t* __restrict__ w, uint16_t* __restrict__ y,
@@ -435,9 +435,8 @@ int nv_gemm_rows(nv_context* c, const void* x, const void* w, void* y, int m, in
     if (n / kTileN < cus_of(c) && m <= 16) {  // too few 16-column tiles to fill the GPU
         if (m <= 8) launch_narrow<8>(c, xb, wb, yb, m, n, k);
         else launch_narrow<16>(c, xb, wb, yb, m, n, k);
-    } else if (n / kTileN >= cus_of(c) && k <= 2048) {  // enough tiles to fill the GPU with 4-wave blocks
-        if (k == 1024) launch_rows_plain<4, 8>(c, xb, wb, yb, m, n, k);
-        else launch_rows_plain<4, 16>(c, xb, wb, yb, m, n, k);
+    } else if (nvr::gemm_stream_fits(c, x, w, y, m, n, k)) {
+        nvr::launch_gemm_stream(c, xb, wb, yb, m, n, k);
     } else {
         switch (k) {
             case 1024: launch_rows_plain<16, 2>(c, xb, wb, yb, m, n, k); break;

@@ -64,13 +64,6 @@ __device__ __forceinline__ float fold8(const float* w) {
     return ((w[0] + w[4]) + (w[2] + w[6])) + ((w[1] + w[5]) + (w[3] + w[7]));
 }
 
-// Byte address in LDS of a pointer into shared memory.
-template <typename T>
-__device__ __forceinline__ uint32_t lds_address(const T* p) {
-    using Lds = __attribute__((address_space(3))) const T*;
-    return static_cast<uint32_t>(reinterpret_cast<uintptr_t>((Lds)p));
-}
-
 // nvr_expf for x <= 0 or NaN, with its bits: the same polynomial, and 2^k
 // applied as 2^(k + 64) (exact, k >= -159) times 2^-64 (the one rounding), so
 // neither branch nor select remains but the one below -110.

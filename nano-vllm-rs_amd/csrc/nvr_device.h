@@ -57,6 +57,13 @@ __device__ __forceinline__ uint4 pack8_split(const float* f) {
                       pack_bf16x2_split(f[4], f[5]), pack_bf16x2_split(f[6], f[7]));
 }
 
+// Byte address in LDS of a pointer into shared memory.
+template <typename T>
+__device__ __forceinline__ uint32_t lds_address(const T* p) {
+    using Lds = __attribute__((address_space(3))) const T*;
+    return static_cast<uint32_t>(reinterpret_cast<uintptr_t>((Lds)p));
+}
+
 // Streaming 16-byte accesses (non-temporal hint on the global load/store) for
 // data each launch touches exactly once; on MI355X they keep the caches for
 // the reused operands and raise copy bandwidth by roughly 7-40% per kernel.

@@ -43,6 +43,11 @@ void launch_attention_tiles(nv_context* c, const uint16_t* q, const uint16_t* k,
                             const int* s, const int* t, uint16_t* o, int rows, int qh, int kvh, int bs, int blocks,
                             int stride, int batch, int max_context);
 
+// nv_gemm's few-row form over a wide weight (gemm_stream.hip): whether the call
+// takes it, and its launch.
+bool gemm_stream_fits(const nv_context* c, const void* x, const void* w, const void* y, int m, int n, int k);
+void launch_gemm_stream(nv_context* c, const uint16_t* x, const uint16_t* w, uint16_t* y, int m, int n, int k);
+
 // Status of the most recent launch on this thread.
 inline int launch_status() { return hip_status(hipGetLastError(), "HIP kernel launch"); }
 

@@ -189,6 +189,11 @@ void nv_graph_destroy(nv_context* c, void* graph) {
 
 int nv_gemm(nv_context* c, const void* x, const void* w, void* y, int m, int n, int k) {
     NVR_ACTIVATE(c);
+    if (nvr::gemm_stream_fits(c, x, w, y, m, n, k)) {
+        nvr::launch_gemm_stream(c, static_cast<const uint16_t*>(x), static_cast<const uint16_t*>(w),
+                                static_cast<uint16_t*>(y), m, n, k);
+        return nvr::launch_status();
+    }
     const float alpha = 1.0f, beta = 0.0f;
     // Row-major Y[m,n] = X[m,k] W[n,k]^T is column-major Y'[n,m] = A' B with
     // A = W seen as column-major [k,n] (lda = k, transposed) and B = X seen as

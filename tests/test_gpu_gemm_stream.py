@@ -1,0 +1,30 @@
+"""The few-row GEMM over a wide weight (nv_gemm and nv_gemm_rows from as many
+16-column tiles as CUs) against the float64 product: one and two row tiles with
+ragged last ones, both k, one tile a block and ragged numbers of tiles, more
+units than the ring's slots, and equal bits from launch to launch."""
+import numpy as np
+import pytest
+
+import oracle as ora
+from helpers import assert_bits_equal
+from test_gpu_kernels import _gemm_bound, down, f32_of, up
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("m", [1, 15, 16, 17, 32])
+@pytest.mark.parametrize("k", [1024, 2048])
+@pytest.mark.parametrize("extra", [0, 1, 255, 700])
+def test_gemm_stream_within_bound(gpu, m, k, extra):
+    n = 16 * (gpu.sm_count() + extra)
+    xa = ora.normal_bf16((m, k), m + k + extra)
+    wa = ora.normal_bf16((n, k), m + k + extra + 1, 0.0, 0.05)
+    x, w, y = up(gpu, xa), up(gpu, wa), up(gpu, np.full((m + 1, n), 0x7FC0, np.uint16))
+    gpu.gemm(x, w, y, m, n, k)
+    got = down(y, np.uint16, (m + 1, n)).copy()
+    assert (got[m] == 0x7FC0).all()  # nothing past the last row
+    want, bound = _gemm_bound(xa, wa)
+    assert np.all(np.abs(f32_of(got[:m]).astype(np.float64) - want) <= bound)
+    for call in (gpu.gemm, gpu.gemm_rows):
+        call(x, w, y, m, n, k)
+        assert_bits_equal(down(y, np.uint16, (m + 1, n))[:m], got[:m])
