@@ -25,7 +25,7 @@
 //      bytes of token tok(m) = 4 (m % 4) + m / 4, d = 32 j .. 32 j + 31: the A
 //      operands of all 32 chains. The permuted tokens make result register r
 //      of lane group a the score of token 4 r + a, which is the operand layout
-//      of phase 3 as it stands. The first kChunk tiles' scores go to LDS.
+//      of phase 3 as it stands. The first CHUNK tiles' scores go to LDS.
 //   2. Row maxima; p = exp(score - max). A wave's tiles 2w, 2w + 1 (mod 16) are
 //      threads 32 w .. 32 w + 31 and 128 + 32 w .. of the reference's block
 //      sum, so the sum's chains and its first five levels stay in the wave.
@@ -35,15 +35,20 @@
 // in phase 2 rather than keep them.
 //
 // Measured on MI355X against one block per row (attention.hip): 8 prompts of
-// 1024 rows in all 80.4 -> 33.3 us, one 1021-token prompt 280 -> 82 us, 1024
-// rows at positions 3072 .. 4095 1627 -> 560 us (54 TFLOP/s of the 140 that the
-// fp32 FMAs reach; the rest is the tree, the exponentials and the second
-// scoring of long contexts).
+// 1024 rows in all 80.4 -> 29.3 us, one 1021-token prompt 280 -> 68.6 us, 1024
+// rows at positions 3072 .. 4095 1627 -> 518 us (58 TFLOP/s of the 140 that the
+// fp32 FMAs reach; the rest is the tree, the exponentials, the second scoring of
+// long contexts and, in short prompts, each block's chain of memory round trips).
 //
-// Masked tokens may hold anything (an Inf or NaN times a zero p, or a -0 sum,
-// must not change a row that does not see them), so tiles that some row sees
-// only in part run their value chains on the VALU with the row's own mask.
+// Masked tokens may hold anything, and must not change a row that does not see
+// them. Their p is +0, so in a tile that some row sees only in part they add a
+// zero of either sign: that changes nothing unless the row's value is itself a
+// zero (-0 + +0), or the token holds an Inf or NaN (0 x Inf). Either way the
+// tile's result is a zero or NaN in that row, and such a tile is done again on
+// the VALU, token by token with the row's own mask (8 prompts of 1024 rows in
+// all, where every block has such tiles: 29.3 us, 34.0 when all of them go that way).
 #include "../../include/nano_hip.h"
+#include "nvr_attention.h"
 #include "nvr_device.h"
 #include "nvr_internal.h"
 
@@ -56,20 +61,21 @@ constexpr int kThreads = 256, kWaves = 4;
 constexpr int kDim = 128;
 constexpr int kRows = 16;    // (token, head) rows per block
 constexpr int kTokens = 16;  // tokens per tile
-constexpr int kChunk = 64;   // tiles whose probabilities LDS holds (64 KB: two blocks per CU)
 constexpr int kMaxTiles = 4096 / kTokens;
 
 __device__ __forceinline__ f32x4_t mfma(float a, float b, f32x4_t c) {
     return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
 }
 
-__global__ __launch_bounds__(kThreads, 2) void attention_tiles(
+// CHUNK = tiles whose probabilities LDS holds (1 KB each); BLOCKS = blocks per CU.
+template <int CHUNK, int BLOCKS>
+__global__ __launch_bounds__(kThreads, BLOCKS) void attention_tiles(
     const uint16_t* __restrict__ q, const uint16_t* __restrict__ kc, const uint16_t* __restrict__ vc,
     const int* __restrict__ positions, const int* __restrict__ seqs, const int* __restrict__ tables,
     uint16_t* __restrict__ out, int rows, int qh, int kvh, int bs, int blocks, int stride, int batch, int max_context,
     int hg_shift, int row_tiles) {
     extern __shared__ __align__(16) unsigned char smem[];
-    f32x4_t* probs = reinterpret_cast<f32x4_t*>(smem);  // [kChunk][64 lanes]
+    f32x4_t* probs = reinterpret_cast<f32x4_t*>(smem);  // [CHUNK][64 lanes]
     __shared__ int tile_row[kMaxTiles];                 // physical token row of each tile's first token, or -1
     __shared__ float red_max[kWaves][kRows];
     __shared__ float red_sum[2 * kWaves][kRows];
@@ -164,7 +170,7 @@ __global__ __launch_bounds__(kThreads, 2) void attention_tiles(
                 load_k(kb, tile_of(s + 2));
 #pragma unroll
                 for (int r = 0; r < 4; ++r) m = fmaxf(m, sc[r]);
-                if (t < kChunk) probs[t * kWave + lane] = sc;
+                if (t < CHUNK) probs[t * kWave + lane] = sc;
             };
             for (int s = 0; tile_of(s) < tiles; s += 2) {
                 step(kA, s);
@@ -180,14 +186,14 @@ __global__ __launch_bounds__(kThreads, 2) void attention_tiles(
 
         float sums[2][2][4] = {};           // the reference's thread sums of this wave's tiles (mod 16)
         f32x4_t o0 = {0, 0, 0, 0}, o1 = {0, 0, 0, 0};
-        for (int c0 = 0; c0 < tiles; c0 += kChunk) {
-            const int c1 = min(tiles, c0 + kChunk);
+        for (int c0 = 0; c0 < tiles; c0 += CHUNK) {
+            const int c1 = min(tiles, c0 + CHUNK);
             // ---- 2. probabilities of the chunk ----
             auto prob = [&](f32x4_t sc, int t, float (&sum)[4]) {
                 f32x4_t p;
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
-                    p[r] = finite ? nvr::nvr_expf(sc[r] - m) : 0.0f;
+                    p[r] = finite ? nvr::exp_nonpositive(sc[r] - m) : 0.0f;
                     sum[r] += p[r];
                 }
                 probs[(t - c0) * kWave + lane] = p;
@@ -221,60 +227,80 @@ __global__ __launch_bounds__(kThreads, 2) void attention_tiles(
             __syncthreads();
 
             // ---- 3. values of the chunk ----
-            const int f1 = min(full, c1);
             auto load_v = [&](uint32_t (&v)[4], int t) {
                 const uint16_t* base = vcol + int64_t(max(place(t), 0)) * token_stride + 32 * wave + 2 * n;
 #pragma unroll
                 for (int r = 0; r < 4; ++r)
                     v[r] = *reinterpret_cast<const uint32_t*>(base + (4 * r + a) * int(token_stride));
             };
-            auto values = [&](const uint32_t (&v)[4], int t) {
-                if (place(t) < 0) return;  // an invalid block adds no term
-                const f32x4_t p = probs[(t - c0) * kWave + lane];
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    o0 = mfma(nvr::bf16_lo(v[r]), p[r], o0);
-                    o1 = mfma(nvr::bf16_hi(v[r]), p[r], o1);
-                }
-            };
-            if (c0 < f1) {
-                uint32_t vA[4], vB[4], vC[4], vD[4];
-                load_v(vA, c0);
-                load_v(vB, c0 + 1);
-                load_v(vC, c0 + 2);
-                for (int t = c0; t < f1; t += 4) {
-                    load_v(vD, t + 3);
-                    values(vA, t);
-                    load_v(vA, t + 4);
-                    if (t + 1 < f1) values(vB, t + 1);
-                    load_v(vB, t + 5);
-                    if (t + 2 < f1) values(vC, t + 2);
-                    load_v(vC, t + 6);
-                    if (t + 3 < f1) values(vD, t + 3);
-                }
-            }
-            // Tiles that some row sees in part: token by token, each row masked by its own context.
-            for (int t = max(full, c0); t < c1; ++t) {
-                const int ph = place(t);
-                if (ph < 0) continue;
-                const uint16_t* base = vcol + int64_t(ph) * token_stride + 32 * wave + 8 * a;
-                uint4 v[kTokens];
-#pragma unroll
-                for (int i = 0; i < kTokens; ++i) v[i] = *reinterpret_cast<const uint4*>(base + i * int(token_stride));
+            // Token by token, each row masked by its own context.
+            auto masked = [&](int t) {
+                const uint16_t* base = vcol + int64_t(place(t)) * token_stride + 32 * wave + 8 * a;
                 const float* pt = reinterpret_cast<const float*>(probs + (t - c0) * kWave);
-#pragma unroll
-                for (int i = 0; i < kTokens; ++i) {
-                    if (t * kTokens + i >= ctx_max) break;  // uniform
+                const int end = min(kTokens, ctx_max - t * kTokens);
+#pragma unroll 1
+                for (int i = 0; i < end; ++i) {
                     const float p = pt[(16 * (i & 3) + n) * 4 + (i >> 2)];
                     const bool sees = t * kTokens + i < ctx;
                     float f[8];
-                    nvr::unpack8(v[i], f);
+                    nvr::unpack8(*reinterpret_cast<const uint4*>(base + i * int(token_stride)), f);
 #pragma unroll
                     for (int r = 0; r < 4; ++r) {
                         const float x = __builtin_fmaf(p, f[2 * r], o0[r]), y = __builtin_fmaf(p, f[2 * r + 1], o1[r]);
                         o0[r] = sees ? x : o0[r];
                         o1[r] = sees ? y : o1[r];
                     }
+                }
+            };
+            auto chains = [&](const uint32_t (&v)[4], int t, f32x4_t& x, f32x4_t& y) {
+                const f32x4_t p = probs[(t - c0) * kWave + lane];
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    x = mfma(nvr::bf16_lo(v[r]), p[r], x);
+                    y = mfma(nvr::bf16_hi(v[r]), p[r], y);
+                }
+            };
+            auto values = [&](const uint32_t (&v)[4], int t) {
+                if (place(t) >= 0) chains(v, t, o0, o1);  // an invalid block adds no term
+            };
+            const int f1 = min(full, c1);
+            uint32_t vA[4], vB[4], vC[4], vD[4];
+            load_v(vA, c0);
+            load_v(vB, c0 + 1);
+            load_v(vC, c0 + 2);
+            int t = c0;
+            for (; t + 3 < f1; t += 4) {
+                load_v(vD, t + 3);
+                values(vA, t);
+                load_v(vA, t + 4);
+                values(vB, t + 1);
+                load_v(vB, t + 5);
+                values(vC, t + 2);
+                load_v(vC, t + 6);
+                values(vD, t + 3);
+            }
+            // The last few, and the tiles that some row sees only in part.
+            for (; t < c1; ++t) {
+                load_v(vD, t + 3);
+                if (place(t) >= 0) {
+                    f32x4_t x = o0, y = o1;
+                    chains(vA, t, x, y);
+                    bool lost = false;
+#pragma unroll
+                    for (int r = 0; r < 4; ++r)
+                        lost |= !(__builtin_fabsf(x[r]) > 0.0f) | !(__builtin_fabsf(y[r]) > 0.0f);
+                    if (t >= full && __ballot(lost && active) != 0) {
+                        masked(t);
+                    } else {
+                        o0 = x;
+                        o1 = y;
+                    }
+                }
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    vA[r] = vB[r];
+                    vB[r] = vC[r];
+                    vC[r] = vD[r];
                 }
             }
             if (c1 < tiles) __syncthreads();  // the next chunk overwrites the probabilities
@@ -325,9 +351,21 @@ void launch_attention_tiles(nv_context* c, const uint16_t* q, const uint16_t* k,
     int shift = 0;
     while (shift < 4 && ratio % (2 << shift) == 0) ++shift;
     const int per = kRows >> shift, row_tiles = (rows + per - 1) / per;
-    hipLaunchKernelGGL(attention_tiles, dim3(unsigned(row_tiles) * unsigned(qh >> shift)), dim3(kThreads),
-                       sizeof(f32x4_t) * kChunk * kWave, c->stream, q, k, v, p, s, t, o, rows, qh, kvh, bs, blocks,
-                       stride, batch, max_context, shift, row_tiles);
+    const unsigned grid = unsigned(row_tiles) * unsigned(qh >> shift);
+    auto launch = [&](auto kernel, int chunk) {
+        hipLaunchKernelGGL(kernel, dim3(grid), dim3(kThreads), sizeof(f32x4_t) * chunk * kWave, c->stream, q, k, v, p, s,
+                           t, o, rows, qh, kvh, bs, blocks, stride, batch, max_context, shift, row_tiles);
+    };
+    // Three blocks a CU hide more of each other's latency than two, and score more
+    // of a long context twice (48 tiles are 768 tokens): with three per CU to fill
+    // them 1021 tokens take 68.6 against 73.0 us, 2 x 512 44.1 against 50.3, 1024 at
+    // 3072 518 against 525 (8 x 128 29.3 against 28.4). A launch of at most one
+    // block per CU keeps 2304 tokens' scores instead: 64 tokens at 2000 91.7 against
+    // 103 us.
+    const unsigned cus = c->cu_count > 0 ? unsigned(c->cu_count) : 256u;
+    if (grid > 2 * cus) launch(attention_tiles<48, 3>, 48);
+    else if (grid > cus) launch(attention_tiles<64, 2>, 64);
+    else launch(attention_tiles<144, 1>, 144);
 }
 
 }  // namespace nvr

@@ -37,6 +37,14 @@ def test_tiles_context_edges(gpu, first, n):
     _attention_case(gpu, 330 + n, pos, seqs, 4, 2, 128, 256, 1, 16, 4096)
 
 
+@pytest.mark.parametrize("rows,first", [(600, 300), (600, 762), (300, 1000), (40, 2290)])
+def test_tiles_chunk_edges_by_launch_size(gpu, rows, first):
+    """With 2 kv heads of 8 q heads a launch has a block a row: more than two per CU keep 768 tokens'
+    probabilities, more than one 1024, fewer 2304; contexts below and across each."""
+    pos, seqs = _rows([(first, rows)])
+    _attention_case(gpu, 340 + rows, pos, seqs, 16, 2, 128, 256, 1, 10, 2560)
+
+
 def test_tiles_rows_in_any_order(gpu):
     """Rows of three sequences interleaved and out of order, decode rows among them."""
     rng = np.random.default_rng(350)
