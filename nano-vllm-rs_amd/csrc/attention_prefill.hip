@@ -17,7 +17,7 @@
 // a row-by-row kernel reads every K and V row from LDS and widens it once per
 // query row, here once per 16.
 //
-// Layout. A block of four waves owns 16 rows: TR = 16 >> hg_shift consecutive
+// Layout. A block of four waves (eight in small launches) owns 16 rows: TR = 16 >> hg_shift consecutive
 // batch rows x HG = 1 << hg_shift q heads of one kv head. Rows of several
 // sequences are processed one sequence at a time (the others masked).
 //   1. Scores, transposed (M = tokens, N = rows): wave w takes tiles of 16
@@ -57,7 +57,7 @@ namespace {
 using nvr::kWave;
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
 
-constexpr int kThreads = 256, kWaves = 4;
+constexpr int kPairs = 8;    // tile pairs (mod 16 tiles) whose thread sums are the reference's warps
 constexpr int kDim = 128;
 constexpr int kRows = 16;    // (token, head) rows per block
 constexpr int kTokens = 16;  // tokens per tile
@@ -67,9 +67,12 @@ __device__ __forceinline__ f32x4_t mfma(float a, float b, f32x4_t c) {
     return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
 }
 
-// CHUNK = tiles whose probabilities LDS holds (1 KB each); BLOCKS = blocks per CU.
-template <int CHUNK, int BLOCKS>
-__global__ __launch_bounds__(kThreads, BLOCKS) void attention_tiles(
+// CHUNK = tiles whose probabilities LDS holds (1 KB each); WAVES = 4 or 8;
+// SIMD_WAVES = waves per SIMD that the registers are to allow. With eight waves
+// each takes one tile pair in eight and, in phase 3, one of the two
+// instructions e.
+template <int CHUNK, int WAVES, int SIMD_WAVES>
+__global__ __launch_bounds__(WAVES * kWave, SIMD_WAVES) void attention_tiles(
     const uint16_t* __restrict__ q, const uint16_t* __restrict__ kc, const uint16_t* __restrict__ vc,
     const int* __restrict__ positions, const int* __restrict__ seqs, const int* __restrict__ tables,
     uint16_t* __restrict__ out, int rows, int qh, int kvh, int bs, int blocks, int stride, int batch, int max_context,
@@ -77,8 +80,10 @@ __global__ __launch_bounds__(kThreads, BLOCKS) void attention_tiles(
     extern __shared__ __align__(16) unsigned char smem[];
     f32x4_t* probs = reinterpret_cast<f32x4_t*>(smem);  // [CHUNK][64 lanes]
     __shared__ int tile_row[kMaxTiles];                 // physical token row of each tile's first token, or -1
-    __shared__ float red_max[kWaves][kRows];
-    __shared__ float red_sum[2 * kWaves][kRows];
+    __shared__ float red_max[WAVES][kRows];
+    __shared__ float red_sum[kPairs][kRows];
+    constexpr int G = kPairs / WAVES;   // tile pairs (mod 16 tiles) per wave
+    constexpr bool BOTH = WAVES == 4;   // a wave runs both instructions e
 
     const int lane = threadIdx.x & (kWave - 1), wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
     const int n = lane & 15, a = lane >> 4;  // row of the tile; lane group
@@ -96,7 +101,8 @@ __global__ __launch_bounds__(kThreads, BLOCKS) void attention_tiles(
     const bool valid = exists && seq_n >= 0 && seq_n < batch && ctx64 >= 1 && ctx64 <= max_context &&
                        ctx64 <= int64_t(stride) * bs;
     const int64_t row_head = int64_t(exists ? row : 0) * qh + head;
-    uint16_t* dst = out + row_head * kDim + 32 * wave + 8 * a;
+    const int wd = BOTH ? wave : wave >> 1, e = BOTH ? 0 : wave & 1;  // dimensions 32 wd ..; (one) instruction
+    uint16_t* dst = out + row_head * kDim + 32 * wd + 8 * a;
     if (exists && !valid) *reinterpret_cast<uint4*>(dst) = make_uint4(0, 0, 0, 0);
 
     float qf[32];  // q[32 a + c]: operand B of chain c
@@ -125,8 +131,8 @@ __global__ __launch_bounds__(kThreads, BLOCKS) void attention_tiles(
         const int tiles = (ctx_max + kTokens - 1) / kTokens, full = ctx_min / kTokens;
         if (int(threadIdx.x) < tiles) {
             const int t0 = int(threadIdx.x) * kTokens, lb = t0 / bs;
-            const int e = tables[int64_t(seq) * stride + lb];
-            tile_row[threadIdx.x] = e >= 0 && e < blocks ? e * bs + (t0 - lb * bs) : -1;
+            const int entry = tables[int64_t(seq) * stride + lb];
+            tile_row[threadIdx.x] = entry >= 0 && entry < blocks ? entry * bs + (t0 - lb * bs) : -1;
         }
         __syncthreads();
 
@@ -155,8 +161,8 @@ __global__ __launch_bounds__(kThreads, BLOCKS) void attention_tiles(
                 s[r] = ok && t * kTokens + 4 * r + a < ctx ? dot[r] * kScale : -__builtin_inff();
             return s;
         };
-        // Wave-tile s of this wave: pairs 2w, 2w + 1 of every eight tiles.
-        auto tile_of = [&](int s) { return 8 * (s >> 1) + 2 * wave + (s & 1); };
+        // Wave-tile s of this wave: the pair 2w, 2w + 1 of every 2 WAVES tiles.
+        auto tile_of = [&](int s) { return 2 * WAVES * (s >> 1) + 2 * wave + (s & 1); };
 
         // ---- 1. scores and row maxima ----
         float m = -__builtin_inff();
@@ -181,10 +187,11 @@ __global__ __launch_bounds__(kThreads, BLOCKS) void attention_tiles(
         m = fmaxf(m, nvr::xor_lane(m, 32));
         if (a == 0) red_max[wave][n] = m;
         __syncthreads();
-        m = fmaxf(fmaxf(red_max[0][n], red_max[1][n]), fmaxf(red_max[2][n], red_max[3][n]));
+#pragma unroll
+        for (int w = 0; w < WAVES; ++w) m = fmaxf(m, red_max[w][n]);
         const bool finite = __builtin_isfinite(m);
 
-        float sums[2][2][4] = {};           // the reference's thread sums of this wave's tiles (mod 16)
+        float sums[G][2][4] = {};           // the reference's thread sums of this wave's tiles (mod 16)
         f32x4_t o0 = {0, 0, 0, 0}, o1 = {0, 0, 0, 0};
         for (int c0 = 0; c0 < tiles; c0 += CHUNK) {
             const int c1 = min(tiles, c0 + CHUNK);
@@ -199,21 +206,21 @@ __global__ __launch_bounds__(kThreads, BLOCKS) void attention_tiles(
                 probs[(t - c0) * kWave + lane] = p;
             };
             if (c0 == 0) {
-                for (int s = 0; tile_of(s) < c1; s += 4) {
+                for (int s = 0; tile_of(s) < c1; s += 2 * G) {
 #pragma unroll
-                    for (int u = 0; u < 4; ++u) {
+                    for (int u = 0; u < 2 * G; ++u) {
                         const int t = tile_of(s + u);
                         if (t < c1) prob(probs[t * kWave + lane], t, sums[u >> 1][u & 1]);
                     }
                 }
             } else {
-                const int s0 = c0 / kWaves;
+                const int s0 = c0 / WAVES;
                 uint4 kA[4], kB[4];
                 load_k(kA, tile_of(s0));
                 load_k(kB, tile_of(s0 + 1));
-                for (int s = s0; tile_of(s) < c1; s += 4) {
+                for (int s = s0; tile_of(s) < c1; s += 2 * G) {
 #pragma unroll
-                    for (int u = 0; u < 4; ++u) {
+                    for (int u = 0; u < 2 * G; ++u) {
                         const int t = tile_of(s + u);
                         uint4(&kb)[4] = u & 1 ? kB : kA;
                         if (t < c1) {
@@ -228,14 +235,14 @@ __global__ __launch_bounds__(kThreads, BLOCKS) void attention_tiles(
 
             // ---- 3. values of the chunk ----
             auto load_v = [&](uint32_t (&v)[4], int t) {
-                const uint16_t* base = vcol + int64_t(max(place(t), 0)) * token_stride + 32 * wave + 2 * n;
+                const uint16_t* base = vcol + int64_t(max(place(t), 0)) * token_stride + 32 * wd + 2 * n;
 #pragma unroll
                 for (int r = 0; r < 4; ++r)
                     v[r] = *reinterpret_cast<const uint32_t*>(base + (4 * r + a) * int(token_stride));
             };
             // Token by token, each row masked by its own context.
             auto masked = [&](int t) {
-                const uint16_t* base = vcol + int64_t(place(t)) * token_stride + 32 * wave + 8 * a;
+                const uint16_t* base = vcol + int64_t(place(t)) * token_stride + 32 * wd + 8 * a;
                 const float* pt = reinterpret_cast<const float*>(probs + (t - c0) * kWave);
                 const int end = min(kTokens, ctx_max - t * kTokens);
 #pragma unroll 1
@@ -246,9 +253,12 @@ __global__ __launch_bounds__(kThreads, BLOCKS) void attention_tiles(
                     nvr::unpack8(*reinterpret_cast<const uint4*>(base + i * int(token_stride)), f);
 #pragma unroll
                     for (int r = 0; r < 4; ++r) {
-                        const float x = __builtin_fmaf(p, f[2 * r], o0[r]), y = __builtin_fmaf(p, f[2 * r + 1], o1[r]);
+                        const float x = __builtin_fmaf(p, e ? f[2 * r + 1] : f[2 * r], o0[r]);
                         o0[r] = sees ? x : o0[r];
-                        o1[r] = sees ? y : o1[r];
+                        if constexpr (BOTH) {
+                            const float y = __builtin_fmaf(p, f[2 * r + 1], o1[r]);
+                            o1[r] = sees ? y : o1[r];
+                        }
                     }
                 }
             };
@@ -256,8 +266,8 @@ __global__ __launch_bounds__(kThreads, BLOCKS) void attention_tiles(
                 const f32x4_t p = probs[(t - c0) * kWave + lane];
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
-                    x = mfma(nvr::bf16_lo(v[r]), p[r], x);
-                    y = mfma(nvr::bf16_hi(v[r]), p[r], y);
+                    x = mfma(nvr::bf16_hi(v[r] << (e ? 0 : 16)), p[r], x);
+                    if constexpr (BOTH) y = mfma(nvr::bf16_hi(v[r]), p[r], y);
                 }
             };
             auto values = [&](const uint32_t (&v)[4], int t) {
@@ -288,7 +298,7 @@ __global__ __launch_bounds__(kThreads, BLOCKS) void attention_tiles(
                     bool lost = false;
 #pragma unroll
                     for (int r = 0; r < 4; ++r)
-                        lost |= !(__builtin_fabsf(x[r]) > 0.0f) | !(__builtin_fabsf(y[r]) > 0.0f);
+                        lost |= !(__builtin_fabsf(x[r]) > 0.0f) || (BOTH && !(__builtin_fabsf(y[r]) > 0.0f));
                     if (t >= full && __ballot(lost && active) != 0) {
                         masked(t);
                     } else {
@@ -310,25 +320,31 @@ __global__ __launch_bounds__(kThreads, BLOCKS) void attention_tiles(
         // Tile pair (2w, 2w + 1): offset 16 between the two tiles, 8 and 4
         // between registers r, 2 and 1 between lane groups a.
 #pragma unroll
-        for (int g = 0; g < 2; ++g) {
+        for (int g = 0; g < G; ++g) {
             float x[4];
 #pragma unroll
             for (int r = 0; r < 4; ++r) x[r] = sums[g][0][r] + sums[g][1][r];
             float s = (x[0] + x[2]) + (x[1] + x[3]);
             s += nvr::xor_lane(s, 32);
             s += nvr::xor_lane(s, 16);
-            if (a == 0) red_sum[4 * g + wave][n] = s;
+            if (a == 0) red_sum[WAVES * g + wave][n] = s;
         }
         __syncthreads();
         const float den = ((red_sum[0][n] + red_sum[4][n]) + (red_sum[2][n] + red_sum[6][n])) +
                           ((red_sum[1][n] + red_sum[5][n]) + (red_sum[3][n] + red_sum[7][n]));
-        float o[8];
+        if constexpr (BOTH) {
+            float o[8];
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            o[2 * r] = den > 0.0f ? o0[r] / den : 0.0f;
-            o[2 * r + 1] = den > 0.0f ? o1[r] / den : 0.0f;
+            for (int r = 0; r < 4; ++r) {
+                o[2 * r] = den > 0.0f ? o0[r] / den : 0.0f;
+                o[2 * r + 1] = den > 0.0f ? o1[r] / den : 0.0f;
+            }
+            if (active) *reinterpret_cast<uint4*>(dst) = nvr::pack8(o);
+        } else {
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+                if (active) dst[2 * r + e] = nvr::f32_to_bf16(den > 0.0f ? o0[r] / den : 0.0f);
         }
-        if (active) *reinterpret_cast<uint4*>(dst) = nvr::pack8(o);
         if (todo != 0) __syncthreads();  // the next sequence reuses the LDS arrays
     }
 }
@@ -352,20 +368,20 @@ void launch_attention_tiles(nv_context* c, const uint16_t* q, const uint16_t* k,
     while (shift < 4 && ratio % (2 << shift) == 0) ++shift;
     const int per = kRows >> shift, row_tiles = (rows + per - 1) / per;
     const unsigned grid = unsigned(row_tiles) * unsigned(qh >> shift);
-    auto launch = [&](auto kernel, int chunk) {
-        hipLaunchKernelGGL(kernel, dim3(grid), dim3(kThreads), sizeof(f32x4_t) * chunk * kWave, c->stream, q, k, v, p, s,
+    auto launch = [&](auto kernel, int chunk, int waves) {
+        hipLaunchKernelGGL(kernel, dim3(grid), dim3(unsigned(waves * kWave)), sizeof(f32x4_t) * chunk * kWave, c->stream, q, k, v, p, s,
                            t, o, rows, qh, kvh, bs, blocks, stride, batch, max_context, shift, row_tiles);
     };
     // Three blocks a CU hide more of each other's latency than two, and score more
     // of a long context twice (48 tiles are 768 tokens): with three per CU to fill
     // them 1021 tokens take 68.6 against 73.0 us, 2 x 512 44.1 against 50.3, 1024 at
     // 3072 518 against 525 (8 x 128 29.3 against 28.4). A launch of at most one
-    // block per CU keeps 2304 tokens' scores instead: 64 tokens at 2000 91.7 against
-    // 103 us.
+    // block per CU keeps 2304 tokens' scores instead, and has eight waves a block:
+    // 64 tokens at 2000 103 -> 91.7 -> 69.7 us, one prompt of 256 16.5 -> 14.9.
     const unsigned cus = c->cu_count > 0 ? unsigned(c->cu_count) : 256u;
-    if (grid > 2 * cus) launch(attention_tiles<48, 3>, 48);
-    else if (grid > cus) launch(attention_tiles<64, 2>, 64);
-    else launch(attention_tiles<144, 1>, 144);
+    if (grid > 2 * cus) launch(attention_tiles<48, 4, 3>, 48, 4);
+    else if (grid > cus) launch(attention_tiles<64, 4, 2>, 64, 4);
+    else launch(attention_tiles<144, 8, 2>, 144, 8);
 }
 
 }  // namespace nvr
