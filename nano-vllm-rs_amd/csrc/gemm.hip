@@ -264,18 +264,21 @@ void launch_rows(nv_context* c, const uint16_t* x, const uint16_t* res, uint16_t
 // MFMA, and the partial tiles are summed through LDS in wave order. It serves
 // what neither gemm_narrow (fewer 16-column tiles than CUs, at most 16 rows)
 // nor gemm_stream (at least as many tiles, k 1024 or 2048) takes, with 16 waves
-// of loads in flight per tile.
-template <int WAVES, int STEPS, int MT>
+// of loads in flight per tile. From 17 rows a block's bytes are mostly X (32 rows
+// against COLS of W, at about 40 GB/s a CU), so with fewer tiles than CUs a tile
+// is 8 columns, the lanes of the other 8 repeating them: 32 rows of n 1024 8.1 ->
+// 7.6 us at k 2048, 11.2 -> 10.4 at 3072; 4 columns take 7.9 and 10.6.
+template <int WAVES, int STEPS, int MT, int COLS>
 __global__ __launch_bounds__(WAVES * 64) void gemm_rows(const uint16_t* __restrict__ x,
                                                         const uint16_t* __restrict__ w, uint16_t* __restrict__ y,
                                                         int m, int n, int k) {
     __shared__ float red[WAVES][MT][256];
     const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
-    const int n0 = blockIdx.x * kTileN;
+    const int n0 = blockIdx.x * COLS;
     const int kb = wave * (32 * STEPS) + 8 * (lane / 16);
     uint4 wv[STEPS], xv[MT][STEPS];
 #pragma unroll
-    for (int s = 0; s < STEPS; ++s) wv[s] = nvr::load_stream(w + int64_t(n0 + lane % 16) * k + kb + 32 * s);
+    for (int s = 0; s < STEPS; ++s) wv[s] = nvr::load_stream(w + int64_t(n0 + lane % COLS) * k + kb + 32 * s);
 #pragma unroll
     for (int t = 0; t < MT; ++t) {
         const int row = t * 16 + lane % 16;
@@ -299,12 +302,12 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_rows(const uint16_t* __restri
 #pragma unroll
         for (int r = 0; r < 4; ++r) red[wave][t][(4 * (lane / 16) + r) * 16 + lane % 16] = acc[t][r];
     __syncthreads();
-    for (int idx = threadIdx.x; idx < MT * 256; idx += WAVES * 64) {
-        const int t = idx / 256, e = idx % 256, row = t * 16 + e / 16;
+    for (int idx = threadIdx.x; idx < MT * 16 * COLS; idx += WAVES * 64) {
+        const int row = idx / COLS, t = row / 16, e = row % 16 * 16 + idx % COLS;
         float sum = red[0][t][e];
 #pragma unroll
         for (int q = 1; q < WAVES; ++q) sum += red[q][t][e];
-        if (row < m) y[int64_t(row) * n + n0 + e % 16] = nvr::f32_to_bf16(sum);
+        if (row < m) y[int64_t(row) * n + n0 + idx % COLS] = nvr::f32_to_bf16(sum);
     }
 }
 
@@ -377,8 +380,13 @@ void launch_narrow(nv_context* c, const uint16_t* x, const uint16_t* w, uint16_t
 template <int WAVES, int STEPS>
 void launch_rows_plain(nv_context* c, const uint16_t* x, const uint16_t* w, uint16_t* y, int m, int n, int k) {
     const dim3 grid(unsigned(n / kTileN)), block(WAVES * 64);
-    if (m <= 16) hipLaunchKernelGGL((gemm_rows<WAVES, STEPS, 1>), grid, block, 0, c->stream, x, w, y, m, n, k);
-    else hipLaunchKernelGGL((gemm_rows<WAVES, STEPS, 2>), grid, block, 0, c->stream, x, w, y, m, n, k);
+    if (m <= 16)
+        hipLaunchKernelGGL((gemm_rows<WAVES, STEPS, 1, 16>), grid, block, 0, c->stream, x, w, y, m, n, k);
+    else if (n / kTileN >= cus_of(c))
+        hipLaunchKernelGGL((gemm_rows<WAVES, STEPS, 2, 16>), grid, block, 0, c->stream, x, w, y, m, n, k);
+    else
+        hipLaunchKernelGGL((gemm_rows<WAVES, STEPS, 2, 8>), dim3(unsigned(n / 8)), block, 0, c->stream, x, w, y, m, n,
+                           k);
 }
 
 template <bool SILU>
@@ -413,6 +421,20 @@ int launch_rms_gemm(nv_context* c, const void* x, const void* residual, void* re
 }
 
 }  // namespace
+
+namespace nvr {
+
+// nv_gemm's calls that nv_gemm_rows' kernels serve better than the library: on
+// MI355X n 1024 at 16 rows 8.3 -> 4.5 us (k 2048) and 9.3 -> 6.0 (k 3072), at 32
+// rows 8.5 -> 7.6 (k 2048). At 32 rows and k 3072 the library wins (7.7 against 10.4).
+bool gemm_rows_fits(const nv_context* c, const void* x, const void* w, int m, int n, int k) {
+    const bool few = m <= 16 && (k == 1024 || k == 2048 || k == 3072 || k == 4096);
+    const bool more = m <= 32 && (k == 1024 || k == 2048);
+    return m >= 1 && (few || more) && n > 0 && n % kTileN == 0 && n / kTileN < cus_of(c) && aligned(x, 16) &&
+           aligned(w, 16);
+}
+
+}  // namespace nvr
 
 extern "C" {
 

@@ -48,6 +48,9 @@ void launch_attention_tiles(nv_context* c, const uint16_t* q, const uint16_t* k,
 bool gemm_stream_fits(const nv_context* c, const void* x, const void* w, const void* y, int m, int n, int k);
 void launch_gemm_stream(nv_context* c, const uint16_t* x, const uint16_t* w, uint16_t* y, int m, int n, int k);
 
+// nv_gemm's calls that take nv_gemm_rows' kernels (gemm.hip).
+bool gemm_rows_fits(const nv_context* c, const void* x, const void* w, int m, int n, int k);
+
 // Status of the most recent launch on this thread.
 inline int launch_status() { return hip_status(hipGetLastError(), "HIP kernel launch"); }
 

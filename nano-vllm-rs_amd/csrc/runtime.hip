@@ -194,6 +194,7 @@ int nv_gemm(nv_context* c, const void* x, const void* w, void* y, int m, int n, 
                                 static_cast<uint16_t*>(y), m, n, k);
         return nvr::launch_status();
     }
+    if (nvr::gemm_rows_fits(c, x, w, m, n, k)) return nv_gemm_rows(c, x, w, y, m, n, k);
     const float alpha = 1.0f, beta = 0.0f;
     // Row-major Y[m,n] = X[m,k] W[n,k]^T is column-major Y'[n,m] = A' B with
     // A = W seen as column-major [k,n] (lda = k, transposed) and B = X seen as

@@ -1,4 +1,4 @@
-"""The few-row GEMM over a wide weight (nv_gemm and nv_gemm_rows from as many
+"""The few-row GEMMs: over a wide weight (nv_gemm and nv_gemm_rows from as many
 16-column tiles as CUs) against the float64 product: one and two row tiles with
 ragged last ones, both k, one tile a block and ragged numbers of tiles, more
 units than the ring's slots, and equal bits from launch to launch."""
@@ -28,3 +28,19 @@ def test_gemm_stream_within_bound(gpu, m, k, extra):
     for call in (gpu.gemm, gpu.gemm_rows):
         call(x, w, y, m, n, k)
         assert_bits_equal(down(y, np.uint16, (m + 1, n))[:m], got[:m])
+
+
+@pytest.mark.parametrize("m", [1, 8, 16, 17, 31, 32])
+@pytest.mark.parametrize("n,k", [(16, 1024), (1024, 2048), (1008, 3072), (2032, 1024), (48, 4096)])
+def test_gemm_narrow_within_bound(gpu, m, n, k):
+    """Fewer 16-column tiles than CUs: 8-column tiles from 17 rows, through both entry points."""
+    xa = ora.normal_bf16((m, k), m + n + k)
+    wa = ora.normal_bf16((n, k), m + n + k + 1, 0.0, 0.05)
+    x, w = up(gpu, xa), up(gpu, wa)
+    want, bound = _gemm_bound(xa, wa)
+    for call in (gpu.gemm, gpu.gemm_rows):
+        y = up(gpu, np.full((m + 1, n), 0x7FC0, np.uint16))
+        call(x, w, y, m, n, k)
+        got = down(y, np.uint16, (m + 1, n))
+        assert (got[m] == 0x7FC0).all()
+        assert np.all(np.abs(f32_of(got[:m]).astype(np.float64) - want) <= bound)
