@@ -356,17 +356,34 @@ class Gpu:
 
     def _admit(self, op: str, args) -> None:
         """Checks the tensor arguments of kernel `op` (the module's contract)."""
-        spans = []
+        # Prompt work is launched call by call, so this runs between its kernels: messages are formed, and the
+        # byte ranges compared, only where they are needed (nine tensors 10.3 -> 5.5 us).
+        device, memories = self._device, set()
         for name, buf, width, dims, _ in args:
-            who = f"{op}: argument '{name}'"
-            if buf._memory.device is not self._device:
-                raise ArgumentError("foreign", f"{who} was not allocated by this Gpu")
-            need = byte_count(dims, width)
+            memory = buf._memory
+            if memory.device is not device:
+                raise ArgumentError("foreign", f"{op}: argument '{name}' was not allocated by this Gpu")
+            need = width
+            for d in dims:
+                if not 1 <= d <= INT_MAX:
+                    as_dim(d)  # raises
+                need *= int(d)
             if need > buf._length:
-                raise ArgumentError("extent", f"{who} needs {need} bytes; its view holds {buf._length}")
+                raise ArgumentError("extent", f"{op}: argument '{name}' needs {need} bytes; its view holds "
+                                              f"{buf._length}")
             if buf._offset % width:
-                raise ArgumentError("alignment", f"{who} starts at byte {buf._offset}, not a multiple of {width}")
-            spans.append((buf._memory, buf._offset, buf._offset + need))
+                raise ArgumentError("alignment", f"{op}: argument '{name}' starts at byte {buf._offset}, not a "
+                                                 f"multiple of {width}")
+            memories.add(memory)
+        if len(memories) != len(args):  # some share an allocation
+            self._refuse_overlap(op, args)
+        if self._device.recording is not None:
+            for _, buf, _, _, _ in args:
+                self._device.recording.setdefault(id(buf._memory), buf._memory)
+
+    @staticmethod
+    def _refuse_overlap(op: str, args) -> None:
+        spans = [(buf._memory, buf._offset, buf._offset + byte_count(dims, width)) for _, buf, width, dims, _ in args]
         for i, (name, _, _, _, written) in enumerate(args):
             if not written:
                 continue
@@ -375,12 +392,10 @@ class Gpu:
                 if j != i and other is mem and max(lo, olo) < min(hi, ohi):
                     raise ArgumentError("overlap", f"{op}: written argument '{name}' shares bytes with "
                                                    f"argument '{args[j][0]}'")
-        if self._device.recording is not None:
-            for _, buf, _, _, _ in args:
-                self._device.recording.setdefault(id(buf._memory), buf._memory)
 
     def _call(self, status: int) -> None:
-        check_status(status, self.lib)
+        if status:
+            check_status(status, self.lib)
 
     # -------------------------------------------------------------- GEMM ---
     def gemm(self, x: Buffer, w: Buffer, y: Buffer, m: int, n: int, k: int) -> None:
