@@ -52,6 +52,8 @@
 #include "nvr_device.h"
 #include "nvr_internal.h"
 
+#include <algorithm>
+
 namespace {
 
 using nvr::fold8;
@@ -721,6 +723,33 @@ int check_attention(int rows, int qh, int kvh, int dim, int bs, int blocks, int 
     return 0;
 }
 
+// A grid dimension holds fewer than 2^32 work-items, and blocks here are at most
+// one per (row, q head): larger calls run as several launches over the rows.
+constexpr int64_t kLaunchHeads = int64_t(1) << 23;
+int launch_rows(int rows, int qh) { return int(std::min<int64_t>(rows, kLaunchHeads / qh)); }
+
+void launch_attention(nv_context* c, const uint16_t* q, uint16_t* k, uint16_t* v, const int* p, const int* s,
+                      const int* t, uint16_t* o, int rows, int qh, int kvh, int dim, int bs, int blocks, int stride,
+                      int batch, int max_context) {
+    // The ordered kernels index cache rows in int32.
+    const bool vec =
+        nvr::aligned(q, 16) && nvr::aligned(k, 16) && nvr::aligned(v, 16) && int64_t(blocks) * bs <= 0x7fffffff;
+    if (vec && nvr::aligned(o, 16) && nvr::attention_tiles_fit(rows, dim, bs, batch))
+        nvr::launch_attention_tiles(c, q, k, v, p, s, t, o, rows, qh, kvh, bs, blocks, stride, batch, max_context);
+    else if (vec && dim == 128)
+        launch_dim<128>(c, q, k, v, p, s, t, o, rows, qh, kvh, bs, blocks, stride, batch, max_context);
+    else if (vec && dim == 64)
+        launch_dim<64>(c, q, k, v, p, s, t, o, rows, qh, kvh, bs, blocks, stride, batch, max_context);
+    else if (vec && dim == 32)
+        launch_dim<32>(c, q, k, v, p, s, t, o, rows, qh, kvh, bs, blocks, stride, batch, max_context);
+    else if (vec && dim == 256)
+        launch_ordered<256, 1>(c, q, k, v, p, s, t, o, rows, qh, kvh, bs, blocks, stride, batch, max_context);
+    else
+        hipLaunchKernelGGL(attention_direct, dim3(unsigned(rows), unsigned(qh)), dim3(kThreads),
+                           sizeof(float) * size_t(max_context), c->stream, q, k, v, p, s, t, o, qh, kvh, dim, bs,
+                           blocks, stride, batch, max_context);
+}
+
 }  // namespace
 
 extern "C" int nv_attention(nv_context* c, const void* q, const void* kc, const void* vc, const void* positions,
@@ -728,32 +757,14 @@ extern "C" int nv_attention(nv_context* c, const void* q, const void* kc, const 
                             int bs, int blocks, int stride, int batch, int max_context) {
     NVR_ACTIVATE(c);
     if (int e = check_attention(rows, qh, kvh, dim, bs, blocks, stride, batch, max_context)) return e;
-    auto q16 = static_cast<const uint16_t*>(q);
     auto k16 = static_cast<uint16_t*>(const_cast<void*>(kc));  // read only: this entry point writes no cache
     auto v16 = static_cast<uint16_t*>(const_cast<void*>(vc));
-    auto p32 = static_cast<const int*>(positions);
-    auto s32 = static_cast<const int*>(seqs);
-    auto t32 = static_cast<const int*>(tables);
-    auto o16 = static_cast<uint16_t*>(out);
-    // The ordered kernels index cache rows in int32.
-    const bool vec = nvr::aligned(q, 16) && nvr::aligned(kc, 16) && nvr::aligned(vc, 16) &&
-                     int64_t(blocks) * bs <= 0x7fffffff;
-    if (vec && nvr::aligned(out, 16) && nvr::attention_tiles_fit(rows, qh, kvh, dim, bs, batch))
-        nvr::launch_attention_tiles(c, q16, k16, v16, p32, s32, t32, o16, rows, qh, kvh, bs, blocks, stride, batch,
-                                    max_context);
-    else if (vec && dim == 128)
-        launch_dim<128>(c, q16, k16, v16, p32, s32, t32, o16, rows, qh, kvh, bs, blocks, stride, batch, max_context);
-    else if (vec && dim == 64)
-        launch_dim<64>(c, q16, k16, v16, p32, s32, t32, o16, rows, qh, kvh, bs, blocks, stride, batch, max_context);
-    else if (vec && dim == 32)
-        launch_dim<32>(c, q16, k16, v16, p32, s32, t32, o16, rows, qh, kvh, bs, blocks, stride, batch, max_context);
-    else if (vec && dim == 256)
-        launch_ordered<256, 1>(c, q16, k16, v16, p32, s32, t32, o16, rows, qh, kvh, bs, blocks, stride, batch,
-                               max_context);
-    else
-        hipLaunchKernelGGL(attention_direct, dim3(unsigned(rows), unsigned(qh)), dim3(kThreads),
-                           sizeof(float) * size_t(max_context), c->stream, q16, k16, v16, p32, s32, t32, o16, qh,
-                           kvh, dim, bs, blocks, stride, batch, max_context);
+    const int step = launch_rows(rows, qh);
+    for (int64_t r = 0; r < rows; r += step)
+        launch_attention(c, static_cast<const uint16_t*>(q) + r * qh * dim, k16, v16,
+                         static_cast<const int*>(positions) + r, static_cast<const int*>(seqs) + r,
+                         static_cast<const int*>(tables), static_cast<uint16_t*>(out) + r * qh * dim,
+                         int(std::min<int64_t>(step, rows - r)), qh, kvh, dim, bs, blocks, stride, batch, max_context);
     return nvr::launch_status();
 }
 
@@ -776,12 +787,20 @@ extern "C" int nv_attention_qkv_rope(nv_context* c, const void* qkv, const void*
           nvr::aligned(vc, 16) && nvr::aligned(rope_cache, 16)) ||
         int64_t(blocks) * bs > 0x7fffffff)
         return nvr::fail(-2, "attention_qkv_rope: needs 16-byte aligned tensors and blocks * bs < 2^31");
-    const QkvRopeArgs fa{static_cast<const uint16_t*>(qkv), static_cast<const uint16_t*>(qw),
-                         static_cast<const uint16_t*>(kw), static_cast<const int*>(slots),
-                         static_cast<const float*>(rope_cache), max_positions, eps};
-    launch_dim<128, true>(c, nullptr, static_cast<uint16_t*>(kc), static_cast<uint16_t*>(vc),
-                          static_cast<const int*>(positions), static_cast<const int*>(seqs),
-                          static_cast<const int*>(tables), static_cast<uint16_t*>(out), rows, qh, kvh, bs, blocks,
-                          stride, batch, max_context, fa);
+    const int step = launch_rows(rows, qh);
+    for (int64_t r = 0; r < rows; r += step) {
+        const QkvRopeArgs fa{static_cast<const uint16_t*>(qkv) + r * (qh + 2 * int64_t(kvh)) * dim,
+                             static_cast<const uint16_t*>(qw),
+                             static_cast<const uint16_t*>(kw),
+                             static_cast<const int*>(slots) + r,
+                             static_cast<const float*>(rope_cache),
+                             max_positions,
+                             eps};
+        launch_dim<128, true>(c, nullptr, static_cast<uint16_t*>(kc), static_cast<uint16_t*>(vc),
+                              static_cast<const int*>(positions) + r, static_cast<const int*>(seqs) + r,
+                              static_cast<const int*>(tables), static_cast<uint16_t*>(out) + r * qh * dim,
+                              int(std::min<int64_t>(step, rows - r)), qh, kvh, bs, blocks, stride, batch, max_context,
+                              fa);
+    }
     return nvr::launch_status();
 }

@@ -356,8 +356,8 @@ namespace nvr {
 // Rows of one sequence share a tile's K and V; a batch of one row per sequence
 // would leave 15 of 16 rows masked and walk its sequences one after the other,
 // so the batch must average at least four rows a sequence.
-bool attention_tiles_fit(int rows, int qh, int kvh, int dim, int bs, int batch) {
-    return dim == kDim && bs % kTokens == 0 && rows >= 4 * int64_t(batch) && int64_t(rows) * qh < (int64_t(1) << 31);
+bool attention_tiles_fit(int rows, int dim, int bs, int batch) {
+    return dim == kDim && bs % kTokens == 0 && rows >= 4 * int64_t(batch);
 }
 
 void launch_attention_tiles(nv_context* c, const uint16_t* q, const uint16_t* k, const uint16_t* v, const int* p,

@@ -668,6 +668,19 @@ def test_attention_aligned_tile_paths_other_head_dims(gpu, dim, qh, kvh, bs, abo
     _attention_case(gpu, 270 + dim + bs + above_cus, pos, seqs, qh, kvh, dim, bs, batch, stride, max_context)
 
 
+def test_attention_more_blocks_than_a_grid_dimension_holds(gpu):
+    """2^24 (row, q head) blocks of 256 threads: one block each would be 2^32 work-items in a grid dimension.
+    Every row sees one token, so its heads are that token's V rows."""
+    dim, heads, bs, batch = 32, 32, 8, 4
+    rows = (1 << 19) + 3
+    vc = ora.normal_bf16((batch, bs, heads, dim), 291)
+    tables, seqs = np.array([2, 0, 3, 1], np.int32), (np.arange(rows) % batch).astype(np.int32)
+    got = _attention(gpu, np.zeros((rows, heads, dim), np.uint16), vc, vc, np.zeros(rows, np.int32), seqs, tables, rows,
+                     heads, heads, dim, bs, batch, 1, batch, bs)
+    for s in range(batch):
+        assert (got[s::batch] == vc[tables[s], 0]).all()
+
+
 def test_attention_invalid_rows_and_blocks(gpu):
     """Rows with a bad sequence index or a context beyond max_context or the
     table give zeros; table entries outside [0, blocks) drop their tokens."""
