@@ -113,6 +113,17 @@ struct OrderedLayout {
 // kStreamed is kAligned with the V tiles streamed into LDS slots.
 constexpr int kAnyBs = 0, kPow2 = 1, kAligned = 2, kStreamed = 3;
 
+// Which blocks share a CU: those that lie 256 apart. With a row's head groups
+// side by side these are different rows, so one long row doesn't fill a CU
+// twice; with the rows side by side, CUs that start together take one kv head.
+// Head dim 128, blocks of whole tiles, at most two blocks per CU: 64 rows at
+// 2048 .. 4096 tokens 187 -> 174 us, at 20 8.4 -> 8.0 with the groups first. The
+// rest is faster with the rows first (groups first, then rows first: 16-token
+// blocks, 64 rows at 60 tokens 12.7, 10.9; 256 rows at 1000 147, 141; head dim
+// 256, 32 rows at 1000 75, 65; head dim 32, 64 rows at 1000 28.0, 24.9).
+template <int DIM, int TABLE, bool OCC>
+constexpr bool kGroupsFirst = DIM == 128 && TABLE == kAligned && !OCC;
+
 template <int DIM, int HPB, int TABLE, bool OCC, bool FUSED>
 __global__ __launch_bounds__(kThreads) void attention_ordered(
     const uint16_t* __restrict__ q, uint16_t* __restrict__ kc, uint16_t* __restrict__ vc,
@@ -131,12 +142,11 @@ __global__ __launch_bounds__(kThreads) void attention_ordered(
     __shared__ float red_max[HPB][kWaves];
     __shared__ float red_sum[HPB][2 * kWaves];
 
-    // A CU holds blocks that lie 256 apart: with the head groups in the fastest
-    // place these are different rows, so one long row doesn't fill a CU twice
-    // (64 rows at contexts of 2048 .. 4096: 187 -> 174 us).
-    const int groups = qh / HPB;
-    const int row = blockIdx.x / groups;
-    const int h0 = (blockIdx.x - row * groups) * HPB;
+    int row = blockIdx.x, h0 = blockIdx.y * HPB;
+    if constexpr (kGroupsFirst<DIM, TABLE, OCC>) {
+        row = blockIdx.x / (qh / HPB);
+        h0 = (blockIdx.x - row * (qh / HPB)) * HPB;
+    }
     const int kvhead = h0 / (qh / kvh);
     const int seq = seqs[row];
     const int64_t context64 = int64_t(positions[row]) + 1;
@@ -625,7 +635,7 @@ void launch_layout(nv_context* c, const uint16_t* q, uint16_t* k, uint16_t* v, c
     const int table_entries = (max_context - 1) / bs + 1;
     using L = OrderedLayout<DIM, HPB, OCC>;
     const size_t lds = sizeof(float) * HPB * score_stride + L::kStageBytes + sizeof(int) * table_entries;
-    const dim3 grid(unsigned(rows) * unsigned(qh / HPB));
+    const dim3 grid(unsigned(rows), unsigned(qh / HPB));
     const bool pow2 = (bs & (bs - 1)) == 0;
     const int shift = pow2 ? __builtin_ctz(unsigned(bs)) : 0;
     // kAligned also needs the row's table in one wave (at most 64 entries) and
@@ -644,10 +654,11 @@ void launch_layout(nv_context* c, const uint16_t* q, uint16_t* k, uint16_t* v, c
             return;
         }
     }
+    constexpr bool flat = kGroupsFirst<DIM, kAligned, OCC>;
     if (aligned)
-        hipLaunchKernelGGL((attention_ordered<DIM, HPB, kAligned, OCC, FUSED>), grid, dim3(kThreads), lds, c->stream,
-                           q, k, v, p, s, t, o, qh, kvh, bs, shift, blocks, stride, batch, max_context, score_stride,
-                           fa);
+        hipLaunchKernelGGL((attention_ordered<DIM, HPB, kAligned, OCC, FUSED>), flat ? dim3(grid.x * grid.y) : grid,
+                           dim3(kThreads), lds, c->stream, q, k, v, p, s, t, o, qh, kvh, bs, shift, blocks, stride,
+                           batch, max_context, score_stride, fa);
     else if (pow2)
         hipLaunchKernelGGL((attention_ordered<DIM, HPB, kPow2, OCC, FUSED>), grid, dim3(kThreads), lds, c->stream,
                            q, k, v, p, s, t, o, qh, kvh, bs, shift, blocks, stride, batch, max_context, score_stride,

@@ -750,15 +750,16 @@ def test_attention_aligned_streamed_and_register_tiles(gpu, extra_rows):
 
 
 @pytest.mark.parametrize("rows,bs,seed", [(8, 256, 300), (32, 256, 310), (8, 16, 320), (5, 7, 330), (32, 16, 340),
-                                         (32, 7, 350)])
+                                         (32, 7, 350), (33, 256, 360), (72, 256, 370), (72, 16, 380)])
 def test_attention_qkv_rope_matches_separate_launches(gpu, rows, bs, seed):
     """The fused decode form (q/k norm + RoPE + KV write inside the attention
     launch) against qkv_rope_cached + paged_attention and the oracle: out and
     both caches bit for bit. One row per sequence with the slot its table
     gives; 8 rows take one q head per block, 32 a GQA pair; 256-, 16- and
     7-token blocks cover the three table lookups (register table, shift and
-    divide), each with a GQA pair per block at 32 rows. The last row of the 5-row
-    case has an invalid sequence and slot -1 (zero output, no KV write)."""
+    divide), each with a GQA pair per block at 32 rows. 33 rows are more than one
+    block per CU (of 256), 72 more than two: the register and the three-blocks-per-CU
+    forms of both launches. The last row of the 5-row case has an invalid sequence and slot -1 (zero output, no KV write)."""
     qh, kvh, dim, max_context = 16, 8, 128, 4096
     rng = np.random.default_rng(seed)
     batch, stride = rows, -(-max_context // bs)
