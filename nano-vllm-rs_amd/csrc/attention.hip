@@ -745,7 +745,7 @@ void launch_attention(nv_context* c, const uint16_t* q, uint16_t* k, uint16_t* v
     // The ordered kernels index cache rows in int32.
     const bool vec =
         nvr::aligned(q, 16) && nvr::aligned(k, 16) && nvr::aligned(v, 16) && int64_t(blocks) * bs <= 0x7fffffff;
-    if (vec && nvr::aligned(o, 16) && nvr::attention_tiles_fit(rows, dim, bs, batch))
+    if (vec && nvr::aligned(o, 16) && nvr::attention_tiles_fit(c, rows, qh, kvh, dim, bs, batch, max_context))
         nvr::launch_attention_tiles(c, q, k, v, p, s, t, o, rows, qh, kvh, bs, blocks, stride, batch, max_context);
     else if (vec && dim == 128)
         launch_dim<128>(c, q, k, v, p, s, t, o, rows, qh, kvh, bs, blocks, stride, batch, max_context);

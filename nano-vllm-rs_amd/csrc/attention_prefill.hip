@@ -355,9 +355,25 @@ namespace nvr {
 
 // Rows of one sequence share a tile's K and V; a batch of one row per sequence
 // would leave 15 of 16 rows masked and walk its sequences one after the other,
-// so the batch must average at least four rows a sequence.
-bool attention_tiles_fit(int rows, int dim, int bs, int batch) {
-    return dim == kDim && bs % kTokens == 0 && rows >= 4 * int64_t(batch);
+// so the batch must average at least four rows a sequence (64 sequences of 4 rows
+// at 1000 tokens 175 -> 77 us, 4 of 4 23 -> 73 by the tiles).
+//
+// A tile walks its context alone, in the time of one row or of sixteen, so few
+// rows are better off spread over the CUs. At blocks that attention_decode takes
+// (16 q heads over 8; one row a block, then tiles, us): 8 rows at 64 tokens 5.5,
+// 9.8, at 1024 21, 39, at 4000 72, 153; 32 rows 6.5, 9.9, then 25, 39 and 87, 154.
+// Up to two blocks per CU one sequence still gains at short contexts (64 rows: 8.2,
+// 9.9, then 40, 39 and 144, 154), several, whose K and V are as many times the
+// bytes, don't (8 of 8 rows at 1024: 56, 40). Other block sizes take attention_ordered,
+// which is slower: 16-token blocks, 16 rows 9.5, 9.9, at 2000 70, 68, 32 rows 10.2, 9.9
+// and 79, 69.
+bool attention_tiles_fit(const nv_context* c, int rows, int qh, int kvh, int dim, int bs, int batch,
+                         int max_context) {
+    if (dim != kDim || bs % kTokens != 0 || rows < 4 * int64_t(batch)) return false;
+    const int64_t cus = c->cu_count > 0 ? c->cu_count : 256, heads = int64_t(rows) * qh;
+    if (!attention_decode_fits(bs, kvh, max_context)) return heads > cus;
+    const int64_t row_blocks = (qh / kvh) % 2 == 0 ? heads / 2 : heads;
+    return row_blocks > (batch == 1 ? 2 * cus : cus);
 }
 
 void launch_attention_tiles(nv_context* c, const uint16_t* q, const uint16_t* k, const uint16_t* v, const int* p,

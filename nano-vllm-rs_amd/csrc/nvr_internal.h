@@ -38,7 +38,7 @@ int create_pair_state(nv_context* c);
 // The tile form of nv_attention (attention_prefill.hip): whether the call's
 // shape takes it, and its launch. Needs 16-byte aligned q, caches and out and
 // blocks * bs below 2^31.
-bool attention_tiles_fit(int rows, int dim, int bs, int batch);
+bool attention_tiles_fit(const nv_context* c, int rows, int qh, int kvh, int dim, int bs, int batch, int max_context);
 void launch_attention_tiles(nv_context* c, const uint16_t* q, const uint16_t* k, const uint16_t* v, const int* p,
                             const int* s, const int* t, uint16_t* o, int rows, int qh, int kvh, int bs, int blocks,
                             int stride, int batch, int max_context);

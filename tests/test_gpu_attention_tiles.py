@@ -3,12 +3,14 @@ whole 16-token tiles) against the oracle, bit for bit: head groups, block
 sizes, edges of tiles and of the 1024-token chunks, tiles that hold rows of
 several sequences, invalid rows and blocks, and values that a masked token
 must not let through."""
+import time
+
 import numpy as np
 import pytest
 
 import oracle as ora
 from helpers import assert_bits_equal
-from test_gpu_kernels import _attention, _attention_case
+from test_gpu_kernels import _attention, _attention_case, up
 
 pytestmark = pytest.mark.gpu
 
@@ -83,3 +85,35 @@ def test_tiles_masked_tokens_do_not_leak(gpu):
     assert nan.any() and (want == 0x8000).any() and ((want & 0x7FFF) == 0x7F80).any()
     assert np.array_equal(nan, (got & 0x7FFF) > 0x7F80)  # a NaN's sign and payload are not specified
     assert_bits_equal(np.where(nan, 0, got), np.where(nan, 0, want))
+
+
+def _attention_us(gpu, spans, qh=16, kvh=8, bs=256):
+    """Best time of one launch over zeros, sequences of their own blocks, in a replayed graph of ten."""
+    pos, seqs = _rows(spans)
+    batch, rows, stride = len(spans), len(pos), 4096 // bs
+    blocks = batch * stride
+    q, cache, out = (gpu.alloc(n) for n in (rows * qh * 256, blocks * bs * kvh * 256, rows * qh * 256))
+    for b in (q, cache):
+        b.upload(np.zeros(b.bytes, np.uint8))
+    args = (up(gpu, pos.astype(np.int32)), up(gpu, seqs.astype(np.int32)), up(gpu, np.arange(blocks, dtype=np.int32)))
+
+    def ten():
+        for _ in range(10):
+            gpu.paged_attention(q, cache, cache, *args, out, rows, qh, kvh, 128, bs, blocks, stride, batch, 4096)
+
+    ten()
+    graph, best = gpu.capture(ten), float("inf")
+    for _ in range(20):
+        gpu.sync()
+        start = time.perf_counter()
+        graph.replay()
+        gpu.sync()
+        best = min(best, time.perf_counter() - start)
+    return best * 1e5
+
+
+@pytest.mark.parametrize("rows", [4, 32])
+def test_tiles_leave_few_rows_to_the_decode_kernel(gpu, rows):
+    """A few rows at the end of a long context take no longer as one sequence than as one sequence each. (By
+    the tiles, which walk such a context alone, 154 us against 47 at 4 rows and 158 against 84 at 32.)"""
+    assert _attention_us(gpu, [(4000, rows)]) < 1.3 * _attention_us(gpu, [(4000 + i, 1) for i in range(rows)])
