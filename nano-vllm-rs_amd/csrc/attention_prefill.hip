@@ -18,8 +18,16 @@
 // query row, here once per 16.
 //
 // Layout. A block of four waves (eight in small launches) owns 16 rows: TR = 16 >> hg_shift consecutive
-// batch rows x HG = 1 << hg_shift q heads of one kv head. Rows of several
-// sequences are processed one sequence at a time (the others masked).
+// batch rows x HG = 1 << hg_shift q heads of one kv head. It does the rows of one
+// sequence at a time (the others masked), so a tile of several would take them one
+// after the other, whatever their contexts. Therefore a launch of several sequences
+// has a block more per sequence and head group, ahead of the tiles' blocks: it does
+// the tile where the sequence begins (its rows there), and the tile's block only what
+// goes on from earlier tiles. Blocks find that out from the sequence ids (1 to 2 us):
+// a prompt of 200 rows beside 31 sequences of one row at 4000 tokens 1236 -> 231 us (a
+// block per row 211), at 300 116 -> 23; 1000 rows beside 24 at 4000 1827 -> 254; 32
+// prompts of 5 rows at 300 45 -> 26; 8 prompts of 128 rows, where no tile has two, 24.3
+// -> 24.9. Rows that alternate between sequences still go one after the other.
 //   1. Scores, transposed (M = tokens, N = rows): wave w takes tiles of 16
 //      tokens 2w, 2w + 1, 2w + 8, 2w + 9, ... Lane (m, j) holds 64 contiguous
 //      bytes of token tok(m) = 4 (m % 4) + m / 4, d = 32 j .. 32 j + 31: the A
@@ -62,6 +70,8 @@ constexpr int kDim = 128;
 constexpr int kRows = 16;    // (token, head) rows per block
 constexpr int kTokens = 16;  // tokens per tile
 constexpr int kMaxTiles = 4096 / kTokens;
+// Sequence ids that a launch's blocks of sequences may read in all (4 bytes each, from L2: 128 MB).
+constexpr int64_t kMaxScan = int64_t(1) << 25;
 
 __device__ __forceinline__ f32x4_t mfma(float a, float b, f32x4_t c) {
     return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
@@ -76,34 +86,92 @@ __global__ __launch_bounds__(WAVES * kWave, SIMD_WAVES) void attention_tiles(
     const uint16_t* __restrict__ q, const uint16_t* __restrict__ kc, const uint16_t* __restrict__ vc,
     const int* __restrict__ positions, const int* __restrict__ seqs, const int* __restrict__ tables,
     uint16_t* __restrict__ out, int rows, int qh, int kvh, int bs, int blocks, int stride, int batch, int max_context,
-    int hg_shift, int row_tiles) {
+    int hg_shift, int row_tiles, int seq_blocks) {
     extern __shared__ __align__(16) unsigned char smem[];
     f32x4_t* probs = reinterpret_cast<f32x4_t*>(smem);  // [CHUNK][64 lanes]
     __shared__ int tile_row[kMaxTiles];                 // physical token row of each tile's first token, or -1
     __shared__ float red_max[WAVES][kRows];
     __shared__ float red_sum[kPairs][kRows];
+    __shared__ uint32_t found[WAVES];
     constexpr int G = kPairs / WAVES;   // tile pairs (mod 16 tiles) per wave
     constexpr bool BOTH = WAVES == 4;   // a wave runs both instructions e
+    constexpr int kThreads = WAVES * kWave;
 
     const int lane = threadIdx.x & (kWave - 1), wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
     const int n = lane & 15, a = lane >> 4;  // row of the tile; lane group
     // Consecutive blocks take the head groups of one row tile, so each XCD
     // (blocks go round the eight) sees few kv heads and keeps their K and V in
-    // its L2; the last rows, whose contexts are the longest, start first.
-    const int groups = qh >> hg_shift;
-    const int group = int(blockIdx.x) % groups, tile = row_tiles - 1 - int(blockIdx.x) / groups;
+    // its L2; the last rows, whose contexts are the longest, start first, and the
+    // blocks of sequences before them (those that find nothing to do are gone at once).
+    const int groups = qh >> hg_shift, per = kRows >> hg_shift;
+    const int item = int(blockIdx.x) / groups, group = int(blockIdx.x) % groups;
+    auto row_valid = [&](int s, int64_t ctx) {
+        return s >= 0 && s < batch && ctx >= 1 && ctx <= max_context && ctx <= int64_t(stride) * bs;
+    };
+    const int own = item < seq_blocks ? item : -1;  // the sequence that this block is for, or -1: a tile's block
+    int tile = row_tiles - 1 - (item - seq_blocks);
+    if (own >= 0) {
+        // The sequence's first row: kScan loads a thread in flight.
+        constexpr int kScan = 4;
+        uint32_t first = uint32_t(rows);
+        for (int r0 = int(threadIdx.x); first == uint32_t(rows) && r0 < rows; r0 += kScan * kThreads) {
+            int s[kScan];
+#pragma unroll
+            for (int u = 0; u < kScan; ++u) s[u] = r0 + u * kThreads < rows ? seqs[r0 + u * kThreads] : -1;
+#pragma unroll
+            for (int u = kScan - 1; u >= 0; --u) {
+                const int r = r0 + u * kThreads;
+                if (s[u] == own && row_valid(own, int64_t(positions[r]) + 1)) first = uint32_t(r);
+            }
+        }
+#pragma unroll
+        for (int o = 1; o < kWave; o <<= 1) first = min(first, nvr::xor_lane_bits(first, o));
+        if (lane == 0) found[wave] = first;
+        __syncthreads();
+#pragma unroll
+        for (int w = 0; w < WAVES; ++w) first = min(first, found[w]);
+        if (first == uint32_t(rows)) return;
+        tile = __builtin_amdgcn_readfirstlane(int(first)) / per;
+    }
     const int head = (group << hg_shift) + (n & ((1 << hg_shift) - 1));
     const int kvhead = (group << hg_shift) / (qh / kvh);
-    const int row = tile * (kRows >> hg_shift) + (n >> hg_shift);
+    const int row = tile * per + (n >> hg_shift);
     const bool exists = row < rows;
     const int seq_n = exists ? seqs[row] : -1;
     const int64_t ctx64 = exists ? int64_t(positions[row]) + 1 : 0;
-    const bool valid = exists && seq_n >= 0 && seq_n < batch && ctx64 >= 1 && ctx64 <= max_context &&
-                       ctx64 <= int64_t(stride) * bs;
+    const bool valid = exists && row_valid(seq_n, ctx64);
+    uint32_t todo = uint32_t(__ballot(valid)) & 0xffffu;  // rows still to do (the same in every wave)
+    if (own >= 0) {
+        todo &= uint32_t(__ballot(seq_n == own));
+    } else if (seq_blocks != 0 && todo != 0) {
+        // The tile's first sequence mostly goes on from the row before; of the others, this block does those that an
+        // earlier tile has seen.
+        const int lead = __builtin_amdgcn_readlane(seq_n, __builtin_ctz(todo));
+        const int before = tile * per - 1;
+        const bool goes_on = before >= 0 && seqs[before] == lead && row_valid(lead, int64_t(positions[before]) + 1);
+        const uint32_t rest = goes_on ? todo & ~uint32_t(__ballot(seq_n == lead)) : todo;
+        if (rest != 0) {
+            uint32_t seen = 0;
+            for (int r = int(threadIdx.x); r < tile * per; r += kThreads) {
+                const int s = seqs[r];
+                uint32_t same = 0;
+#pragma unroll
+                for (int i = 0; i < kRows; ++i) same |= uint32_t(s == __builtin_amdgcn_readlane(seq_n, i)) << i;
+                if ((same & rest) != 0 && row_valid(s, int64_t(positions[r]) + 1)) seen |= same;
+            }
+#pragma unroll
+            for (int o = 1; o < kWave; o <<= 1) seen |= nvr::xor_lane_bits(seen, o);
+            if (lane == 0) found[wave] = seen;
+            __syncthreads();
+#pragma unroll
+            for (int w = 0; w < WAVES; ++w) seen |= found[w];
+            todo &= ~rest | uint32_t(__builtin_amdgcn_readfirstlane(int(seen)));
+        }
+    }
     const int64_t row_head = int64_t(exists ? row : 0) * qh + head;
     const int wd = BOTH ? wave : wave >> 1, e = BOTH ? 0 : wave & 1;  // dimensions 32 wd ..; (one) instruction
     uint16_t* dst = out + row_head * kDim + 32 * wd + 8 * a;
-    if (exists && !valid) *reinterpret_cast<uint4*>(dst) = make_uint4(0, 0, 0, 0);
+    if (own < 0 && exists && !valid) *reinterpret_cast<uint4*>(dst) = make_uint4(0, 0, 0, 0);
 
     float qf[32];  // q[32 a + c]: operand B of chain c
 #pragma unroll
@@ -115,7 +183,6 @@ __global__ __launch_bounds__(WAVES * kWave, SIMD_WAVES) void attention_tiles(
     const uint16_t* vcol = vc + int64_t(kvhead) * kDim;
     const int klane = (4 * (n & 3) + (n >> 2)) * int(token_stride) + 32 * a;
 
-    uint32_t todo = uint32_t(__ballot(valid)) & 0xffffu;  // rows still to do (the same in every wave)
     while (todo != 0) {
         const int seq = __builtin_amdgcn_readlane(seq_n, __builtin_ctz(todo));
         const bool active = valid && seq_n == seq;
@@ -382,20 +449,26 @@ void launch_attention_tiles(nv_context* c, const uint16_t* q, const uint16_t* k,
     const int ratio = qh / kvh;
     int shift = 0;
     while (shift < 4 && ratio % (2 << shift) == 0) ++shift;
-    const int per = kRows >> shift, row_tiles = (rows + per - 1) / per;
-    const unsigned grid = unsigned(row_tiles) * unsigned(qh >> shift);
+    const int per = kRows >> shift, row_tiles = (rows + per - 1) / per, groups = qh >> shift;
+    const int seq_blocks = batch > 1 && int64_t(batch) * rows * groups <= kMaxScan ? batch : 0;
+    const unsigned grid = unsigned(row_tiles + seq_blocks) * unsigned(groups);
     auto launch = [&](auto kernel, int chunk, int waves) {
-        hipLaunchKernelGGL(kernel, dim3(grid), dim3(unsigned(waves * kWave)), sizeof(f32x4_t) * chunk * kWave, c->stream, q, k, v, p, s,
-                           t, o, rows, qh, kvh, bs, blocks, stride, batch, max_context, shift, row_tiles);
+        hipLaunchKernelGGL(kernel, dim3(grid), dim3(unsigned(waves * kWave)),
+                           sizeof(f32x4_t) * chunk * kWave, c->stream, q, k, v, p, s, t, o, rows, qh, kvh, bs, blocks,
+                           stride, batch, max_context, shift, row_tiles, seq_blocks);
     };
     // Three blocks a CU hide more of each other's latency than two, and score more
     // of a long context twice (48 tiles are 768 tokens): with three per CU to fill
     // them 1021 tokens take 68.6 against 73.0 us, 2 x 512 44.1 against 50.3, 1024 at
     // 3072 518 against 525 (8 x 128 29.3 against 28.4). A launch of at most one
     // block per CU keeps 2304 tokens' scores instead, and has eight waves a block:
-    // 64 tokens at 2000 103 -> 91.7 -> 69.7 us, one prompt of 256 16.5 -> 14.9.
+    // 64 tokens at 2000 103 -> 91.7 -> 69.7 us, one prompt of 256 16.5 -> 14.9. The
+    // sequences' blocks count there, where a second round would cost as much as the
+    // first (8 prompts of 30 rows 9.4 us, by eight waves 15.1), but not above (some do
+    // nothing; 64 sequences of 8 rows at 1000 tokens 128 us, by three blocks a CU 139).
+    const unsigned tiles = unsigned(row_tiles) * unsigned(groups);
     const unsigned cus = c->cu_count > 0 ? unsigned(c->cu_count) : 256u;
-    if (grid > 2 * cus) launch(attention_tiles<48, 4, 3>, 48, 4);
+    if (tiles > 2 * cus) launch(attention_tiles<48, 4, 3>, 48, 4);
     else if (grid > cus) launch(attention_tiles<64, 4, 2>, 64, 4);
     else launch(attention_tiles<144, 8, 2>, 144, 8);
 }

@@ -87,6 +87,33 @@ def test_tiles_masked_tokens_do_not_leak(gpu):
     assert_bits_equal(np.where(nan, 0, got), np.where(nan, 0, want))
 
 
+MIXED = [(300, 1), (0, 70), (512, 1), (31, 1), (0, 1), (40, 2), (200, 3), (17, 15), (0, 33), (100, 1), (0, 150)]
+
+
+@pytest.mark.parametrize("qh,kvh", [(1, 1), (4, 2), (8, 2), (6, 2), (16, 8), (16, 1), (32, 1)])
+@pytest.mark.parametrize("bs", [16, 256])
+@pytest.mark.parametrize("order", ["sorted", "shuffled"])
+def test_tiles_of_several_sequences(gpu, qh, kvh, bs, order):
+    """One to sixteen rows a tile, one to eight sequences in it, at sequences whose first rows are first in their
+    tile or not; sorted, and with every tile holding several sequences that others hold too. Some rows are invalid,
+    first rows of their sequence among them, and sequence 4 has none that is valid."""
+    pos, seqs = _rows(MIXED * (1 if qh > 2 else 2))
+    seqs = seqs % len(MIXED)
+    pos[[1, 73, 74, 75, 130]], seqs[[80, 99, 150]] = [-1, 600, -7, 4096, 5000], [-1, len(MIXED), 99]
+    if order == "shuffled":
+        mixed = np.random.default_rng(380).permutation(len(pos))
+        pos, seqs = pos[mixed], seqs[mixed]
+    _attention_case(gpu, 381 + qh + bs, pos, seqs, qh, kvh, 128, bs, len(MIXED), -(-600 // bs), 600)
+
+
+def test_tiles_of_too_many_sequences_for_blocks_of_their_own(gpu):
+    """600 sequences of 4 rows over 32 heads: their blocks would read more ids than a launch's bound allows, so
+    tiles do all their sequences themselves."""
+    pos, seqs = _rows([(i % 9, 3 + i % 3) for i in range(600)])
+    assert len(pos) * 600 * 32 > 1 << 25
+    _attention_case(gpu, 395, pos, seqs, 32, 32, 128, 16, 600, 1, 16)
+
+
 def _attention_us(gpu, spans, qh=16, kvh=8, bs=256):
     """Best time of one launch over zeros, sequences of their own blocks, in a replayed graph of ten."""
     pos, seqs = _rows(spans)
@@ -117,3 +144,11 @@ def test_tiles_leave_few_rows_to_the_decode_kernel(gpu, rows):
     """A few rows at the end of a long context take no longer as one sequence than as one sequence each. (By
     the tiles, which walk such a context alone, 154 us against 47 at 4 rows and 158 against 84 at 32.)"""
     assert _attention_us(gpu, [(4000, rows)]) < 1.3 * _attention_us(gpu, [(4000 + i, 1) for i in range(rows)])
+
+
+@pytest.mark.parametrize("one,context", [(31, 4000), (7, 2000)])
+def test_tiles_do_not_queue_sequences_of_one_row(gpu, one, context):
+    """Sequences of one row beside a prompt cost about what they cost alone: by tiles that walk their sequences one
+    after the other 1217 us against 81 for 31 rows alone, and 461 against 27 for 7."""
+    alone = [(context, 1)] * one
+    assert _attention_us(gpu, [(0, 200)] + alone) < 4 * _attention_us(gpu, alone)
