@@ -265,9 +265,11 @@ void launch_rows(nv_context* c, const uint16_t* x, const uint16_t* res, uint16_t
 // what neither gemm_narrow (fewer 16-column tiles than CUs, at most 16 rows)
 // nor gemm_stream (at least as many tiles, k 1024 or 2048) takes, with 16 waves
 // of loads in flight per tile. From 17 rows a block's bytes are mostly X (32 rows
-// against COLS of W, at about 40 GB/s a CU), so with fewer tiles than CUs a tile
-// is 8 columns, the lanes of the other 8 repeating them: 32 rows of n 1024 8.1 ->
-// 7.6 us at k 2048, 11.2 -> 10.4 at 3072; 4 columns take 7.9 and 10.6.
+// against COLS of W, at about 40 GB/s a CU), so while that leaves at most a block per
+// CU a tile is 8 columns, the lanes of the other 8 repeating them: 32 rows of n 1024
+// 8.1 -> 7.6 us at k 2048, 11.2 -> 10.4 at 3072; 4 columns take 7.9 and 10.6. Beyond,
+// CUs would read X twice: n 2064 in tiles of 16 and of 8 columns 8.3 and 12.7 us at
+// k 2048, 14.4 and 24.1 at 4096.
 template <int WAVES, int STEPS, int MT, int COLS>
 __global__ __launch_bounds__(WAVES * 64) void gemm_rows(const uint16_t* __restrict__ x,
                                                         const uint16_t* __restrict__ w, uint16_t* __restrict__ y,
@@ -382,7 +384,7 @@ void launch_rows_plain(nv_context* c, const uint16_t* x, const uint16_t* w, uint
     const dim3 grid(unsigned(n / kTileN)), block(WAVES * 64);
     if (m <= 16)
         hipLaunchKernelGGL((gemm_rows<WAVES, STEPS, 1, 16>), grid, block, 0, c->stream, x, w, y, m, n, k);
-    else if (n / kTileN >= cus_of(c))
+    else if (n / 8 > cus_of(c))
         hipLaunchKernelGGL((gemm_rows<WAVES, STEPS, 2, 16>), grid, block, 0, c->stream, x, w, y, m, n, k);
     else
         hipLaunchKernelGGL((gemm_rows<WAVES, STEPS, 2, 8>), dim3(unsigned(n / 8)), block, 0, c->stream, x, w, y, m, n,

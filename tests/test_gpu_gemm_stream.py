@@ -2,6 +2,8 @@
 16-column tiles as CUs) against the float64 product: one and two row tiles with
 ragged last ones, both k, one tile a block and ragged numbers of tiles, more
 units than the ring's slots, and equal bits from launch to launch."""
+import time
+
 import numpy as np
 import pytest
 
@@ -43,4 +45,48 @@ def test_gemm_narrow_within_bound(gpu, m, n, k):
         call(x, w, y, m, n, k)
         got = down(y, np.uint16, (m + 1, n))
         assert (got[m] == 0x7FC0).all()
+        assert np.all(np.abs(f32_of(got[:m]).astype(np.float64) - want) <= bound)
+
+
+def _gemm_us(gpu, call, m, n, k):
+    """Best time of one product over zeros, in a replayed graph of twenty."""
+    x, w, y = (gpu.alloc(2 * size) for size in (m * k, n * k, m * n))
+    for b in (x, w):
+        b.upload(np.zeros(b.bytes, np.uint8))
+
+    def twenty():
+        for _ in range(20):
+            call(x, w, y, m, n, k)
+
+    twenty()
+    graph, best = gpu.capture(twenty), float("inf")
+    for _ in range(20):
+        gpu.sync()
+        start = time.perf_counter()
+        graph.replay()
+        gpu.sync()
+        best = min(best, time.perf_counter() - start)
+    return best * 5e4
+
+
+@pytest.mark.parametrize("k", [2048, 4096])
+def test_gemm_rows_take_one_round_of_blocks(gpu, k):
+    """One 16-column tile more than fit as 8-column tiles, a block per CU, costs little more than the last that fit
+    (in 8-column tiles, two rounds of blocks, half as much again)."""
+    n = 8 * gpu.sm_count()
+    assert _gemm_us(gpu, gpu.gemm_rows, 32, n + 16, k) < 1.3 * _gemm_us(gpu, gpu.gemm_rows, 32, n, k)
+
+
+@pytest.mark.parametrize("m", [17, 32])
+@pytest.mark.parametrize("k", [1024, 2048, 3072, 4096])
+def test_gemm_rows_around_one_round_of_blocks(gpu, m, k):
+    """The last n of 8-column tiles and the first of 16-column ones."""
+    for n in (8 * gpu.sm_count(), 8 * gpu.sm_count() + 16):
+        xa = ora.normal_bf16((m, k), m + n + k)
+        wa = ora.normal_bf16((n, k), m + n + k + 1, 0.0, 0.05)
+        y = up(gpu, np.full((m + 1, n), 0x7FC0, np.uint16))
+        gpu.gemm_rows(up(gpu, xa), up(gpu, wa), y, m, n, k)
+        got = down(y, np.uint16, (m + 1, n))
+        assert (got[m] == 0x7FC0).all()
+        want, bound = _gemm_bound(xa, wa)
         assert np.all(np.abs(f32_of(got[:m]).astype(np.float64) - want) <= bound)
