@@ -426,14 +426,22 @@ int launch_rms_gemm(nv_context* c, const void* x, const void* residual, void* re
 
 namespace nvr {
 
-// nv_gemm's calls that nv_gemm_rows' kernels serve better than the library: on
-// MI355X n 1024 at 16 rows 8.3 -> 4.5 us (k 2048) and 9.3 -> 6.0 (k 3072), at 32
-// rows 8.5 -> 7.6 (k 2048). At 32 rows and k 3072 the library wins (7.7 against 10.4).
+// nv_gemm's calls that nv_gemm_rows' kernels serve better than the library, whose
+// time at these sizes grows with k and hardly with n, where a block here reads all
+// of X for its columns. On MI355X, library and here in us (W cold, n from 256 to 4080,
+// k 1024 to 4096):
+//   up to 8 rows always: n 1024 at k 2048 8.4, 3.9; n 4080 at k 3072 11.2, 9.8;
+//   9 to 16 rows (at 16): n 4080 at k 1024 6.4, 6.3; n 3072 at k 2048 8.6, 8.4 and 3584
+//   8.8, 9.3; n 1920 at k 3072 9.6, 9.3 and 2560 9.7, 11.4; n 2048 at k 4096 11.6, 10.2
+//   and 2560 11.7, 11.9;
+//   17 to 32 rows at k 1024 and 2048 past the sizes where the library is fastest: n
+//   1024 at k 1024 4.5, 4.9 and 1152 5.9, 4.9; n 512 at k 2048 5.5, 7.1 and 640 8.3,
+//   7.1; n 2560 8.7, 8.4. At k 3072 and 32 rows the library takes 7.7 and this 10.4.
 bool gemm_rows_fits(const nv_context* c, const void* x, const void* w, int m, int n, int k) {
-    const bool few = m <= 16 && (k == 1024 || k == 2048 || k == 3072 || k == 4096);
-    const bool more = m <= 32 && (k == 1024 || k == 2048);
-    return m >= 1 && (few || more) && n > 0 && n % kTileN == 0 && n / kTileN < cus_of(c) && aligned(x, 16) &&
-           aligned(w, 16);
+    if (m < 1 || n <= 0 || n % kTileN != 0 || n / kTileN >= cus_of(c) || !aligned(x, 16) || !aligned(w, 16)) return false;
+    if (m <= 8) return k == 1024 || k == 2048 || k == 3072 || k == 4096;
+    if (m <= 16) return k == 1024 || (k == 2048 && n <= 3072) || (k == 3072 && n <= 1920) || (k == 4096 && n <= 2048);
+    return m <= 32 && ((k == 1024 && n >= 1152) || (k == 2048 && n >= 576));
 }
 
 }  // namespace nvr

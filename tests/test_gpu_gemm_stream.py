@@ -77,6 +77,27 @@ def test_gemm_rows_take_one_round_of_blocks(gpu, k):
     assert _gemm_us(gpu, gpu.gemm_rows, 32, n + 16, k) < 1.3 * _gemm_us(gpu, gpu.gemm_rows, 32, n, k)
 
 
+@pytest.mark.parametrize("m,n,k", [(16, 4080, 3072), (16, 3584, 4096), (24, 512, 2048), (32, 256, 2048)])
+def test_gemm_leaves_to_the_library_what_it_does_faster(gpu, m, n, k):
+    """Few rows, but more bytes of X in all the blocks than of W, or products that the library splits over k."""
+    assert _gemm_us(gpu, gpu.gemm, m, n, k) < 0.92 * _gemm_us(gpu, gpu.gemm_rows, m, n, k)
+
+
+@pytest.mark.parametrize("m,n,k", [(16, 3072, 2048), (16, 3088, 2048), (9, 1920, 3072), (16, 1936, 3072),
+                                   (16, 2048, 4096), (16, 2064, 4096), (8, 4080, 4096), (17, 1136, 1024),
+                                   (32, 1152, 1024), (17, 560, 2048), (32, 576, 2048)])
+def test_gemm_around_the_library_s_sizes(gpu, m, n, k):
+    """The last product on either side of each line of the rule."""
+    xa = ora.normal_bf16((m, k), m + n + k)
+    wa = ora.normal_bf16((n, k), m + n + k + 1, 0.0, 0.05)
+    y = up(gpu, np.full((m + 1, n), 0x7FC0, np.uint16))
+    gpu.gemm(up(gpu, xa), up(gpu, wa), y, m, n, k)
+    got = down(y, np.uint16, (m + 1, n))
+    assert (got[m] == 0x7FC0).all()
+    want, bound = _gemm_bound(xa, wa)
+    assert np.all(np.abs(f32_of(got[:m]).astype(np.float64) - want) <= bound)
+
+
 @pytest.mark.parametrize("m", [17, 32])
 @pytest.mark.parametrize("k", [1024, 2048, 3072, 4096])
 def test_gemm_rows_around_one_round_of_blocks(gpu, m, k):
