@@ -189,6 +189,9 @@ void nv_graph_destroy(nv_context* c, void* graph) {
 
 int nv_gemm(nv_context* c, const void* x, const void* w, void* y, int m, int n, int k) {
     NVR_ACTIVATE(c);
+    // The library refuses a null operand of a product that has any; so do the kernels that stand in for it.
+    if (m > 0 && n > 0 && k > 0 && (x == nullptr || w == nullptr || y == nullptr))
+        return nvr::fail(-2, "gemm: x, w and y are required (m %d, n %d, k %d)", m, n, k);
     if (nvr::gemm_stream_fits(c, x, w, y, m, n, k)) {
         nvr::launch_gemm_stream(c, static_cast<const uint16_t*>(x), static_cast<const uint16_t*>(w),
                                 static_cast<uint16_t*>(y), m, n, k);

@@ -48,6 +48,17 @@ def test_gemm_narrow_within_bound(gpu, m, n, k):
         assert np.all(np.abs(f32_of(got[:m]).astype(np.float64) - want) <= bound)
 
 
+@pytest.mark.parametrize("m,n,k", [(8, 8192, 1024), (8, 1024, 2048), (32, 1024, 2048), (64, 1024, 1024)])
+@pytest.mark.parametrize("null", [0, 1, 2])
+def test_gemm_refuses_a_null_operand(gpu, m, n, k, null):
+    """On the host, whichever kernel the shape takes."""
+    buffers = [gpu.alloc(2 * size) for size in (m * k, n * k, m * n)]
+    args = [None if i == null else b.ptr for i, b in enumerate(buffers)]
+    assert gpu.lib.nv_gemm(gpu._device.ctx, *args, m, n, k) == -2
+    assert b"required" in gpu.lib.nv_last_error()
+    gpu.sync()
+
+
 def _gemm_us(gpu, call, m, n, k):
     """Best time of one product over zeros, in a replayed graph of twenty."""
     x, w, y = (gpu.alloc(2 * size) for size in (m * k, n * k, m * n))
