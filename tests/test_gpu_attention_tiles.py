@@ -1,8 +1,9 @@
 """nv_attention's tile form (several rows per sequence, head dim 128, blocks of
 whole 16-token tiles) against the oracle, bit for bit: head groups, block
-sizes, edges of tiles and of the 1024-token chunks, tiles that hold rows of
-several sequences, invalid rows and blocks, and values that a masked token
-must not let through."""
+sizes, edges of tiles and of the chunks, tiles that hold rows of several
+sequences, invalid rows and blocks, and values that a masked token must not let
+through. Launches of few rows, the first tests' among them, take the per-row
+kernels; the others bring enough rows for each size of launch."""
 import time
 
 import numpy as np
@@ -87,11 +88,49 @@ def test_tiles_masked_tokens_do_not_leak(gpu):
     assert_bits_equal(np.where(nan, 0, got), np.where(nan, 0, want))
 
 
+@pytest.mark.parametrize("rows", [264, 1056, 2064])
+def test_tiles_masked_tokens_do_not_leak_in_any_form(gpu, rows):
+    """The same with launches of at most one block per CU (of 256), of at most two and of more: rows at positions 36
+    .. 83 in turn, so every tile has rows that don't see all of its tokens."""
+    qh, kvh, dim, bs, blocks = 4, 2, 128, 16, 8
+    q = ora.normal_bf16((rows, qh, dim), 371, 0.0, 6.0)
+    kc, vc = (ora.normal_bf16((blocks, bs, kvh, dim), seed) for seed in (372, 373))
+    flat = vc.reshape(blocks * bs, kvh, dim)
+    flat[:37, :, 16:24], flat[0, :, 16:24], flat[37:, :, 16:24] = 0x8000, 0x8001, 0x3F80
+    vc[3, 0, :, 40:48], vc[3, 5, :, 48:52], vc[3, 9, :, 52:56] = 0x7F80, 0xFF80, 0x7FC0
+    kc[4, 3, 0, 7], kc[4, 5, 1, 9] = 0x7FC0, 0x7F80
+    tables, seqs = np.arange(blocks, dtype=np.int32), np.zeros(rows, np.int32)
+    pos = (np.arange(rows) % 48 + 36).astype(np.int32)
+    want = ora.attention(q, kc, vc, pos, seqs, tables, rows, qh, kvh, dim, bs, blocks, blocks, 1, 128, threads=8)
+    got = _attention(gpu, q, kc, vc, pos, seqs, tables, rows, qh, kvh, dim, bs, blocks, blocks, 1, 128)
+    nan = (want & 0x7FFF) > 0x7F80
+    assert nan.any() and (want == 0x8000).any() and ((want & 0x7FFF) == 0x7F80).any()
+    assert np.array_equal(nan, (got & 0x7FFF) > 0x7F80)
+    assert_bits_equal(np.where(nan, 0, got), np.where(nan, 0, want))
+
+
+@pytest.mark.parametrize("first,n", [(0, 16), (0, 17), (15, 9), (1007, 40), (1016, 8), (2040, 24), (2290, 40),
+                                     (4079, 17)])
+def test_tiles_context_edges_of_many_rows(gpu, first, n):
+    """Edges of tiles and chunks with enough rows (80 or so, repeated) of 16 heads over 2."""
+    pos, seqs = _rows([(first, n)])
+    pos, seqs = np.tile(pos, -(-66 // n)), np.tile(seqs, -(-66 // n))
+    _attention_case(gpu, 335 + n, pos, seqs, 16, 2, 128, 256, 1, 16, 4096)
+
+
+def test_tiles_invalid_blocks_of_many_rows(gpu):
+    """Table entries outside the cache at the start, in the middle and at the end of contexts."""
+    stride, bs = 5, 64
+    pos, seqs = _rows([(180, 120), (30, 120), (0, 160)])
+    holes = [(1, -1), (3, 3 * stride), (stride + 1, -9), (2 * stride, 3 * stride + 4), (2 * stride + 2, -2)]
+    _attention_case(gpu, 365, pos, seqs, 4, 2, 128, bs, 3, stride, 320, q_std=6.0, holes=holes)
+
+
 MIXED = [(300, 1), (0, 70), (512, 1), (31, 1), (0, 1), (40, 2), (200, 3), (17, 15), (0, 33), (100, 1), (0, 150)]
 
 
 @pytest.mark.parametrize("qh,kvh", [(1, 1), (4, 2), (8, 2), (6, 2), (16, 8), (16, 1), (32, 1)])
-@pytest.mark.parametrize("bs", [16, 256])
+@pytest.mark.parametrize("bs", [16, 48, 256])
 @pytest.mark.parametrize("order", ["sorted", "shuffled"])
 def test_tiles_of_several_sequences(gpu, qh, kvh, bs, order):
     """One to sixteen rows a tile, one to eight sequences in it, at sequences whose first rows are first in their
