@@ -147,10 +147,9 @@ __global__ __launch_bounds__(kThreads) void gemm_stream(const uint16_t* __restri
 
 template <int MT, int KS>
 void launch(nv_context* c, const uint16_t* x, const uint16_t* w, uint16_t* y, int m, int n, int cus) {
-    const int tiles = n / kTileN;
     const size_t lds = kWaves * kRing * kUnitBytes + sizeof(f32x4_t) * 2 * kWaves * MT * kWave;
-    hipLaunchKernelGGL((gemm_stream<MT, KS>), dim3(unsigned(tiles < cus ? tiles : cus)), dim3(kThreads), lds,
-                       c->stream, x, w, y, m, n);
+    hipLaunchKernelGGL((gemm_stream<MT, KS>), dim3(unsigned(cus)), dim3(kThreads), lds, c->stream, x, w,
+                       y, m, n);
 }
 
 }  // namespace
