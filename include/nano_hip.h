@@ -73,7 +73,11 @@ void nv_graph_destroy(nv_context* c, void* graph);
 /* ---------------------------------------------------------------- GEMM ---- */
 
 /* kernels/kernels.cu:98-106 — row-major Y[m,n] = X[m,k] * W[n,k]^T, bf16 in and
- * out, fp32 accumulation, through hipBLAS (src/gpu.rs:535-560). */
+ * out, fp32 accumulation (src/gpu.rs:535-560). hipBLAS, except for products of
+ * at most 32 rows whose n, k and 16-byte aligned x and w one of this library's
+ * own kernels serves faster: there the order of the fp32 sums is that kernel's,
+ * and two calls of one shape at other alignments may differ by fp32 rounding.
+ * Every call repeats its bits. A null operand is refused (-2). */
 int nv_gemm(nv_context* c, const void* x, const void* w, void* y, int m, int n, int k);
 
 /* ------------------------------------------------ fused per-layer kernels ---- */
@@ -109,8 +113,8 @@ int nv_add_rms_gather(nv_context* c, const void* x, const void* residual, const 
  * (src/model.rs:659-678 and :753-770). With residual == NULL, X = RMSNorm(x);
  * otherwise v = x + residual, residual_out <- bf16(v) (a different buffer from
  * residual; may be NULL) and X = RMSNorm(v), both exactly as nv_add_rms.
- * Then y[m, n] = bf16(X W^T) with fp32 accumulation in a fixed order (not
- * hipBLAS's: equal to nv_gemm to fp32 rounding). normed (may be NULL) receives
+ * Then y[m, n] = bf16(X W^T) with fp32 accumulation in a fixed order (its own:
+ * equal to nv_gemm to fp32 rounding). normed (may be NULL) receives
  * X. Limits (else -2): 1 <= m <= 32, n a multiple of 16, k in {512, 1024, 2048},
  * 16-byte aligned tensors. x, residual, residual_out, normed: [m, k];
  * w: [n, k]; y: [m, n]. */

@@ -672,10 +672,11 @@ void launch_layout(nv_context* c, const uint16_t* q, uint16_t* k, uint16_t* v, c
 // Blocks are (row, head group) and each walks its context serially, so when
 // there are more than two blocks per CU the occupancy layout wins (three
 // blocks per CU at 164 VGPRs and 52 KB of LDS for head dim 128 and 4096
-// positions): measured on MI355X, 1024 prefill rows 164 -> 108 us (8 x 128
-// tokens) and 457 -> 348 us (one 1024-token prompt). With at most two per CU
-// the deeper pipelines win (64 x 4096 decode: 200 vs 210 us). FUSED launches
-// (decode batches) keep the default layout.
+// positions): measured on MI355X, one row a sequence, 96 rows at 250 tokens 26.9
+// -> 20.9 us, 256 at 1000 149 -> 141 (128 at 1000, a round and a third of blocks,
+// 82.8 -> 86.8); prompts in 8-token blocks, 8 x 128 tokens 153 -> 97 and one of
+// 1000 423 -> 325. With at most two per CU the deeper pipelines win (64 x 4096
+// decode: 200 vs 210 us). FUSED launches (decode batches) keep the default layout.
 template <int DIM, int HPB, bool FUSED = false>
 void launch_ordered(nv_context* c, const uint16_t* q, uint16_t* k, uint16_t* v, const int* p,
                     const int* s, const int* t, uint16_t* o, int rows, int qh, int kvh, int bs, int blocks,
@@ -685,7 +686,8 @@ void launch_ordered(nv_context* c, const uint16_t* q, uint16_t* k, uint16_t* v, 
     // free, which wins at long contexts (64 rows on 256 CUs at 2048 .. 4096
     // tokens 158 against 174 us, at 1024 48 against 52) but loses at short ones
     // (40 rows at 64 tokens 13.2 against 11.9 us, 128 at 100 28.3 against 25.6),
-    // and the host doesn't know the contexts.
+    // and the arguments don't tell the contexts (a caller that knows its longest
+    // passes the model's limit as max_context all the same).
     if constexpr (DIM == 128) {
         if (groups <= cus && nvr::attention_decode_fits(bs, kvh, max_context)) {
             nvr::launch_attention_decode<HPB, FUSED>(c, q, k, v, p, s, t, o, rows, qh, kvh, bs, blocks, stride, batch,
@@ -712,7 +714,8 @@ void launch_dim(nv_context* c, const uint16_t* q, uint16_t* k, uint16_t* v, cons
     // per block still leaves every block a CU, that wins: twice the blocks on an
     // otherwise idle GPU (head dim 128 on MI355X, 16 rows: 10.3 vs 11.2 us at 250
     // tokens of context, 21.6 vs 22.6 at 1024; 24 rows, more heads than CUs: 29.6
-    // vs 20.7 us at 700).
+    // vs 20.7 us at 700; in 16-token blocks the two are level: 24 rows at 250 15.4
+    // vs 15.6, 31 at 1000 45.0 vs 42.3).
     const int64_t cus = c->cu_count > 0 ? c->cu_count : 256;
     const int64_t pairs_from = DIM == 128 ? cus / 2 + 1 : cus;
     if (DIM <= 128 && (qh / kvh) % 2 == 0 && int64_t(rows) * (qh / 2) >= pairs_from)

@@ -427,11 +427,12 @@ namespace nvr {
 //
 // A tile walks its context alone, in the time of one row or of sixteen, so few
 // rows are better off spread over the CUs. At blocks that attention_decode takes
-// (16 q heads over 8; one row a block, then tiles, us): 8 rows at 64 tokens 5.5,
-// 9.8, at 1024 21, 39, at 4000 72, 153; 32 rows 6.5, 9.9, then 25, 39 and 87, 154.
-// Up to two blocks per CU one sequence still gains at short contexts (64 rows: 8.2,
-// 9.9, then 40, 39 and 144, 154), several, whose K and V are as many times the
-// bytes, don't (8 of 8 rows at 1024: 56, 40). Other block sizes take attention_ordered,
+// (16 q heads over 8; one row a block, then tiles, us): 8 rows at 64 tokens 5.3,
+// 9.8, at 1024 15, 39, at 4000 46, 153; 32 rows 6.1, 9.9, then 18, 39 and 56, 154.
+// Up to two blocks per CU, by attention_ordered, one sequence still gains at short
+// contexts (64 rows: 8.2, 9.9, then 40, 39 and 143, 154); several, whose K and V are
+// as many times the bytes, gain less there (4 prompts of 20 rows 8.4, 9.7) than they
+// lose at others (at 300 tokens 24, 19; 8 of 8 rows at 1024 56, 40). Other block sizes take attention_ordered,
 // which is slower: 16-token blocks, 16 rows 9.5, 9.9, at 2000 70, 68, 32 rows 10.2, 9.9
 // and 79, 69.
 bool attention_tiles_fit(const nv_context* c, int rows, int qh, int kvh, int dim, int bs, int batch,

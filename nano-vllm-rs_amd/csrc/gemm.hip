@@ -438,7 +438,8 @@ namespace nvr {
 //   1024 at k 1024 4.5, 4.9 and 1152 5.9, 4.9; n 512 at k 2048 5.5, 7.1 and 640 8.3,
 //   7.1; n 2560 8.7, 8.4. At k 3072 and 32 rows the library takes 7.7 and this 10.4.
 bool gemm_rows_fits(const nv_context* c, const void* x, const void* w, int m, int n, int k) {
-    if (m < 1 || n <= 0 || n % kTileN != 0 || n / kTileN >= cus_of(c) || !aligned(x, 16) || !aligned(w, 16)) return false;
+    if (m < 1 || n <= 0 || n % kTileN != 0 || n / kTileN >= cus_of(c) || !aligned(x, 16) || !aligned(w, 16))
+        return false;
     if (m <= 8) return k == 1024 || k == 2048 || k == 3072 || k == 4096;
     if (m <= 16) return k == 1024 || (k == 2048 && n <= 3072) || (k == 3072 && n <= 1920) || (k == 4096 && n <= 2048);
     return m <= 32 && ((k == 1024 && n >= 1152) || (k == 2048 && n >= 576));

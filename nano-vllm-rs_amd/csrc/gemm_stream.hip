@@ -19,9 +19,10 @@
 // others go on. The order is fixed, so every launch of a shape gives the same
 // bits.
 //
-// Measured on MI355X against hipBLAS (us; W cold): n 151936, k 1024 at 8 rows
-// 60.8 -> 52.9 and at 32 rows 74.0 -> 59.9 (5.2 TB/s of W); n 4096, k 1024 at 32
-// rows 8.4 -> 4.7; n 6144 8.5 -> 6.0. Four slots a wave instead of three change
+// Measured on MI355X against hipBLAS (us a launch in graphs over three weights of
+// normal values, W cold): n 151936, k 1024 at 8 rows 62.2 -> 53.4 and at 32 rows
+// 75.6 -> 59.8 (5.2 TB/s of W); kernel time in a decode step of 8 rows 57.7 -> 50.3;
+// n 4096, k 1024 at 32 rows 8.4 -> 4.7; n 6144 8.5 -> 6.0. Four slots a wave instead of three change
 // nothing; operands read from memory in their own layout take 58.9 us at one row
 // of n 151936 (here 52) and 118 at 32.
 #include "nvr_device.h"
