@@ -43,8 +43,8 @@
 // in phase 2 rather than keep them.
 //
 // Measured on MI355X against one block per row (attention.hip): 8 prompts of
-// 1024 rows in all 80.4 -> 29.3 us, one 1021-token prompt 280 -> 68.6 us, 1024
-// rows at positions 3072 .. 4095 1627 -> 518 us (58 TFLOP/s of the 140 that the
+// 1024 rows in all 80.7 -> 26.3 us, one 1021-token prompt 280 -> 64.8 us, 1024
+// rows at positions 3072 .. 4095 1627 -> 517 us (58 TFLOP/s of the 140 that the
 // fp32 FMAs reach; the rest is the tree, the exponentials, the second scoring of
 // long contexts and, in short prompts, each block's chain of memory round trips).
 //
